@@ -339,7 +339,7 @@ int LevelAdjoint::forward(double dT, const double* const* U, double* const* Unex
       const long N = blocks_[p]->npts();
       FieldsIn src;
       for (int v = 0; v < NFIELD; ++v) src.p[v] = blocks_[p]->stage_output(3) + v * N;
-      adj_launch_copy_fields(src, as_out(Unext + p * NFIELD), N, s);
+      launch_copy_fields(src, as_out(Unext + p * NFIELD), N, s);
     }
   if (hipGetLastError() != hipSuccess) {
     err_ = "level adjoint forward: kernel launch failed";
@@ -363,7 +363,7 @@ int LevelAdjoint::backward(double dT, const double* const* U, double* const* lam
     const long N = blocks_[p]->npts();
     FieldsOut dst;
     for (int v = 0; v < NFIELD; ++v) dst.p[v] = blocks_[p]->lY() + v * N;
-    adj_launch_copy_fields(as_in(lam + p * NFIELD), dst, N, s);
+    launch_copy_fields(as_in(lam + p * NFIELD), dst, N, s);
   }
   exchange_adjoint(s);
   for (int p = 0; p < np; ++p) {

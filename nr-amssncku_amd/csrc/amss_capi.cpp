@@ -1020,17 +1020,66 @@ int amss_level_copy(amss_level* L, int patch, int list, int field, double* ptr, 
   return 0;
 }
 
+// Whether one kernel of the current device may copy between the level's list
+// (24 consecutive grid functions from f0) and the 24 arrays: all of them whole
+// inside allocations of this device (hipMemcpyAsync checks the same), on 8
+// bytes, none reaching into the list, and no two overlapping when written (24
+// copies in order would leave the last one's values).
+static bool copy_list_one_launch(const double* f0, size_t n, double* const* ptrs, int dir, hipStream_t s) {
+  int dev = 0, sdev = -1;
+  if (hipGetDevice(&dev) != hipSuccess || hipStreamGetDevice(s, &sdev) != hipSuccess || dev != sdev) return false;
+  const uintptr_t bytes = n * sizeof(double), l0 = (uintptr_t)f0, l1 = l0 + 24 * bytes;
+  uintptr_t lo = 0, hi = 0;  // the allocation last looked up
+  uintptr_t a[24];
+  for (int v = 0; v < 24; ++v) {
+    const uintptr_t p = a[v] = (uintptr_t)ptrs[v];
+    if (p % 8 != 0 || (p < l1 && l0 < p + bytes)) return false;
+    if (p >= lo && p + bytes <= hi) continue;
+    hipPointerAttribute_t at;
+    hipDeviceptr_t base = nullptr;
+    size_t size = 0;
+    if (hipPointerGetAttributes(&at, ptrs[v]) != hipSuccess || at.type != hipMemoryTypeDevice || at.device != dev ||
+        hipMemGetAddressRange(&base, &size, (hipDeviceptr_t)ptrs[v]) != hipSuccess) {
+      (void)hipGetLastError();
+      return false;
+    }
+    lo = (uintptr_t)base;
+    hi = lo + size;
+    if (p + bytes > hi) return false;
+  }
+  if (dir == 0) return true;
+  std::sort(a, a + 24);
+  for (int v = 1; v < 24; ++v)
+    if (a[v] < a[v - 1] + bytes) return false;
+  return true;
+}
+
 int amss_level_copy_list(amss_level* L, int patch, int list, double* const* ptrs, int dir) {
   if (!L || !ptrs) return fail(AMSS_ERR_ARG, "amss_level_copy_list: null argument");
   if (list < AMSS_LIST_STATE || list > AMSS_LIST_RHS) return fail(AMSS_ERR_ARG, "amss_level_copy_list: bad list");
   const size_t n = (size_t)L->L->npts(patch);
+  double* f[24];
   for (int v = 0; v < 24; ++v) {
-    double* f = L->L->field(patch, list, v);
-    if (!f || !ptrs[v]) return fail(AMSS_ERR_ARG, "amss_level_copy_list: no such grid function");
+    f[v] = L->L->field(patch, list, v);
+    if (!f[v] || !ptrs[v]) return fail(AMSS_ERR_ARG, "amss_level_copy_list: no such grid function");
+  }
+  hipStream_t s = L->L->stream();
+  if (copy_list_one_launch(f[0], n, ptrs, dir, s)) {
+    FieldsIn src;
+    FieldsOut dst;
+    for (int v = 0; v < 24; ++v) {
+      src.p[v] = dir == 0 ? ptrs[v] : f[v];
+      dst.p[v] = dir == 0 ? f[v] : ptrs[v];
+    }
+    launch_copy_fields(src, dst, (long)n, s);
+    HIPCHK(hipGetLastError());
+    return 0;
+  }
+  for (int v = 0; v < 24; ++v) {
     if (dir == 0)
-      HIPCHK(hipMemcpyAsync(f, ptrs[v], n * sizeof(double), hipMemcpyDeviceToDevice, L->L->stream()));
+      HIPCHK(hipMemcpyAsync(f[v], ptrs[v], n * sizeof(double), hipMemcpyDeviceToDevice, s));
     else
-      HIPCHK(hipMemcpyAsync(ptrs[v], f, n * sizeof(double), hipMemcpyDeviceToDevice, L->L->stream()));
+      HIPCHK(hipMemcpyAsync(ptrs[v], f[v], n * sizeof(double), hipMemcpyDeviceToDevice, s));
   }
   return 0;
 }

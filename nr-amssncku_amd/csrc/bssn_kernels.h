@@ -97,6 +97,9 @@ void launch_sommer_interp(const double* X, const double* Y, const double* Z, con
 void launch_ghost_fill(const FieldsIn& u0, const FieldsOut& out, const Box& box, const Faces& w, int stage,
                        double tinny, int* flag, hipStream_t s);
 void launch_seg_copy(const FieldsIn& src, const FieldsOut& dst, const SegDesc& d, hipStream_t s);
+// 24 grid functions of n points, src -> dst (no two of the 48 arrays may
+// overlap where one is written).
+void launch_copy_fields(const FieldsIn& src, const FieldsOut& dst, long n, hipStream_t s);
 void launch_enforce(const FieldsOut& f, long n, hipStream_t s);
 void launch_lowerbound(double* chi, long n, double tinny, hipStream_t s);
 void launch_rk4_update(const double* f0, double* f1, double* frhs, long n, double dT, int stage, hipStream_t s);
