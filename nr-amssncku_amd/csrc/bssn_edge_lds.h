@@ -144,6 +144,10 @@ struct EdgeLdsEnv : EdgeStencils<ORD, EdgeLdsEnv<ORD, NRM>> {
   __device__ __forceinline__ double rel(int, int di, int dj, int dk, double off) const {
     return (cur() + (lt - kLow))[kLow + di + dj * W::P0 + dk * W::P01] + off;
   }
+  // the window holds +-3 points on every side of the tile, array or not
+  __device__ __forceinline__ double rel_clamped(int v, int di, int dj, int dk, double off) const {
+    return rel(v, di, dj, dk, off);
+  }
   __device__ __forceinline__ double val(int v) const {
     if (g == 0 && in_top(v)) return top[v];
     if (g > 0 && v == group_field(g - 1)) return cur()[lt];
