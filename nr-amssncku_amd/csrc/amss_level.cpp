@@ -532,9 +532,9 @@ int BssnLevel::slot_of(MyList<var>* l) const {
 }
 
 // Device tables of the batched step: patch views, the interior tiles of every
-// patch for each tile shape (whole tiles only; what is left of an interior
-// goes to the direct kernel), the boundary boxes of every patch and the
-// inter-patch exchange boxes.
+// patch for each tile shape (patches with an odd row pitch are launched one
+// by one instead), the boundary boxes of every patch and the inter-patch
+// exchange boxes.
 void BssnLevel::build_batch_tables() {
   const int np = (int)blocks_.size();
   hpd_.clear();
@@ -565,30 +565,29 @@ void BssnLevel::build_batch_tables() {
       }
       box.sy = b.shape[0];
       box.sz = (long)b.shape[0] * b.shape[1];
-      int core[3];
-      for (int a = 0; a < 3; ++a) core[a] = 3 + (box.hi[a] - 3) / T[a] * T[a];
-      // tiles need an even row pitch (16-byte aligned direct loads); a patch
-      // with an odd one is all remainder (direct kernel)
-      if (b.shape[0] % 2 != 0) core[0] = core[1] = core[2] = 3;
-      if (core[0] > 3 && core[1] > 3 && core[2] > 3) {
-        if (b.shape[0] > 65535 || b.shape[1] > 65535 || b.shape[2] > 65535 || pi > 65535) {
-          err_ = "patch too large for the tile list";
-          return;
-        }
-        for (int k = 3; k < core[2]; k += T[2])
-          for (int j = 3; j < core[1]; j += T[1])
-            for (int i = 3; i < core[0]; i += T[0])
-              htiles_[sh].push_back(TileRef{(unsigned short)pi, (unsigned short)i, (unsigned short)j,
-                                            (unsigned short)k});
-      } else {
-        for (int a = 0; a < 3; ++a) core[a] = 3;
+      // the tile list's kernels need an even row pitch (16-byte aligned
+      // direct loads); a patch with an odd one runs in a launch of its own
+      // (and so does one that holds no whole tile and is too long for TileRef)
+      bool empty = false, whole = true;
+      for (int a = 0; a < 3; ++a) {
+        empty = empty || box.hi[a] <= 3;
+        whole = whole && box.hi[a] - 3 >= T[a];
       }
-      for (int a = 0; a < 3; ++a) {  // remainder slab [core[a], hi[a]) along a
-        Box r = box;
-        for (int c = 0; c < a; ++c) r.hi[c] = core[c];
-        r.lo[a] = core[a];
-        if (r.hi[0] > r.lo[0] && r.hi[1] > r.lo[1] && r.hi[2] > r.lo[2]) rem_[sh].push_back({pi, r});
+      const bool large = b.shape[0] > 65535 || b.shape[1] > 65535 || b.shape[2] > 65535 || pi > 65535;
+      if (b.shape[0] % 2 != 0 || (large && !whole)) {
+        if (!empty) rem_[sh].push_back({pi, box});
+        continue;
       }
+      if (large) {
+        err_ = "patch too large for the tile list";
+        return;
+      }
+      // whole and partial tiles: the kernel masks the points past the interior
+      for (int k = 3; k < box.hi[2]; k += T[2])
+        for (int j = 3; j < box.hi[1]; j += T[1])
+          for (int i = 3; i < box.hi[0]; i += T[0])
+            htiles_[sh].push_back(TileRef{(unsigned short)pi, (unsigned short)i, (unsigned short)j,
+                                          (unsigned short)k});
     }
     if ((long)htiles_[sh].size() > (1L << 31) - 1) { err_ = "too many tiles"; return; }
     if (!htiles_[sh].empty()) {
@@ -728,13 +727,11 @@ int BssnLevel::StepBatched(double dT, bool want_res) {
     AuxOut aux;
     for (int a = 0; a < 18; ++a) aux.gam[a] = nullptr;
     for (int a = 0; a < 6; ++a) aux.ric[a] = nullptr;
-    Rk4Param Rd = R;
-    Rd.variant = 0;
     for (const auto& pr : rem_[sh]) {
       const Block& b = *blocks_[pr.first];
       for (int a = 0; a < 7; ++a) aux.res[a] = b.fgfs[kResidualBase + a];
       launch_rk4(list_in(b, in), list_in(b, StateList), list_out(b, RHSList), list_out(b, out), aux, pr.second,
-                 coef_[pr.first], Rd, gauge_, res, dflag_, false, stream_, true);
+                 coef_[pr.first], R, gauge_, res, dflag_, false, stream_, true);
     }
     if (bc_ != AMSS_BC_FROZEN_GHOSTS || gw_ < 3) {
       for (int pi = 0; pi < np; ++pi) {
@@ -840,8 +837,6 @@ int BssnLevel::autotune(double* ms, int nms) {
   AuxOut aux;
   for (int a = 0; a < 18; ++a) aux.gam[a] = nullptr;
   for (int a = 0; a < 6; ++a) aux.ric[a] = nullptr;
-  Rk4Param Rd = R;
-  Rd.variant = 0;
   for (int sh = 0; sh < kNumTileShapes; ++sh)
     for (int gm = 0; gm < 3; ++gm)
       for (int rm = 0; rm < 2; ++rm, ++c) {
@@ -857,7 +852,7 @@ int BssnLevel::autotune(double* ms, int nms) {
             const Block& b = *blocks_[pr.first];
             for (int a = 0; a < 7; ++a) aux.res[a] = b.fgfs[kResidualBase + a];
             launch_rk4(list_in(b, StateList), list_in(b, StateList), list_out(b, RHSList),
-                       list_out(b, SynchList_pre), aux, pr.second, coef_[pr.first], Rd, gauge_, false, dflag_, false,
+                       list_out(b, SynchList_pre), aux, pr.second, coef_[pr.first], R, gauge_, false, dflag_, false,
                        stream_, true);
           }
           RCHK(hipEventRecord(e1, stream_));

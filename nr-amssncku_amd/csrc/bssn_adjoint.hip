@@ -42,16 +42,18 @@ __global__ void __launch_bounds__(kRhsThreads) __attribute__((amdgpu_waves_per_e
 rhs_k_lds_kernel(FieldsIn in, FieldsOut out, Box box, Coef C) {
   using Tl = LdsTile<kLdsTX, kLdsTY, kLdsTZ>;
   __shared__ __attribute__((aligned(16))) double tiles[kLdsBuffers * Tl::NPAD];
-  const int tx = threadIdx.x % kLdsTX, ty = tile_row((threadIdx.x / kLdsTX) % kLdsTY, kLdsTY),
-            tz = threadIdx.x / (kLdsTX * kLdsTY);
+  int tx, ty, tz;
+  Tl::point((int)threadIdx.x, tx, ty, tz);
   const int gx = (box.hi[0] - box.lo[0]) / kLdsTX, gy = (box.hi[1] - box.lo[1]) / kLdsTY;
   const int b = xcd_spread(blockIdx.x, gridDim.x);
   const int i0 = box.lo[0] + (b % gx) * kLdsTX, j0 = box.lo[1] + ((b / gx) % gy) * kLdsTY;
   const int k0 = box.lo[2] + (b / (gx * gy)) * kLdsTZ;
   const long p = (i0 + tx) + (long)(j0 + ty) * box.sy + (long)(k0 + tz) * box.sz;
+  const BufIo io{(unsigned)p * 8u, (unsigned)p * 8u, (unsigned)(box.n[0] * box.n[1] * box.n[2]) * 8u};
   lds_double* t0 = (lds_double*)tiles;
-  LdsEnv<kLdsTX, kLdsTY, kLdsTZ> E{in, in, C, t0, t0 + (kLdsBuffers / 2) * Tl::NPAD, p,
-                                  (tx + 3) + Tl::LX * ((ty + 3) + Tl::LY * (tz + 3)),
+  LdsEnv<kLdsTX, kLdsTY, kLdsTZ> E{in, in, C, t0, t0 + (kLdsBuffers / 2) * Tl::NPAD,
+                                  io,
+                                  Tl::lds_index(tx, ty, tz, (int)box.sz),
                                   (int)((i0 - 3) + (j0 - 3) * box.sy + (k0 - 3) * box.sz), (int)box.sy, (int)box.sz,
                                   box.n[0] * box.n[1] * box.n[2], (int)threadIdx.x};
   E.prologue();
@@ -123,14 +125,15 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))
 adj_feature_lds_kernel(FieldsIn in, FieldsIn lam, double* feat, long fs, Box box, Coef C) {
   using Tl = LdsTile<kLdsTX, kLdsTY, kLdsTZ>;
   __shared__ __attribute__((aligned(16))) double tiles[kLdsBuffers * Tl::NPAD];
-  const int tx = threadIdx.x % kLdsTX, ty = tile_row((threadIdx.x / kLdsTX) % kLdsTY, kLdsTY),
-            tz = threadIdx.x / (kLdsTX * kLdsTY);
+  int tx, ty, tz;
+  Tl::point((int)threadIdx.x, tx, ty, tz);
   const int gx = (box.hi[0] - box.lo[0]) / kLdsTX, gy = (box.hi[1] - box.lo[1]) / kLdsTY;
   const int b = xcd_spread(blockIdx.x, gridDim.x);
   const int i0 = box.lo[0] + (b % gx) * kLdsTX, j0 = box.lo[1] + ((b / gx) % gy) * kLdsTY;
   const int k0 = box.lo[2] + (b / (gx * gy)) * kLdsTZ;
   const long p = (i0 + tx) + (long)(j0 + ty) * box.sy + (long)(k0 + tz) * box.sz;
   const int N = box.n[0] * box.n[1] * box.n[2];
+  const BufIo io{(unsigned)p * 8u, (unsigned)p * 8u, (unsigned)N * 8u};
   lds_double* t0 = (lds_double*)tiles;
   // lam and beta at the point, loaded before the first halo loads (so no wait
   // for them stalls on those): every field's upwind term needs all three beta
@@ -140,8 +143,9 @@ adj_feature_lds_kernel(FieldsIn in, FieldsIn lam, double* feat, long fs, Box box
 #pragma unroll
   for (int a = 0; a < 3; ++a) bp[a] = in.p[BETAX + a][p];
   __builtin_amdgcn_sched_barrier(0);
-  LdsEnv<kLdsTX, kLdsTY, kLdsTZ> E{in, in, C, t0, t0 + (kLdsBuffers / 2) * Tl::NPAD, p,
-                                  (tx + 3) + Tl::LX * ((ty + 3) + Tl::LY * (tz + 3)),
+  LdsEnv<kLdsTX, kLdsTY, kLdsTZ> E{in, in, C, t0, t0 + (kLdsBuffers / 2) * Tl::NPAD,
+                                  io,
+                                  Tl::lds_index(tx, ty, tz, (int)box.sz),
                                   (int)((i0 - 3) + (j0 - 3) * box.sy + (k0 - 3) * box.sz), (int)box.sy, (int)box.sz, N,
                                   (int)threadIdx.x};
   E.prologue();

@@ -7,29 +7,32 @@
 namespace amss {
 
 // One tile of the list: the same LDS-staged point computation as
-// rk4_lds_kernel, with the fields of the tile's patch addressed through the
+// rk4_lds_kernel (partial tiles included), with the fields of the tile's patch addressed through the
 // slab and the role slots.
 template <int GAUGE, int STAGE, bool CO, int TX, int TY, int TZ>
 __device__ __forceinline__ void tile_body(const PatchDesc* __restrict__ P, const TileRef& r, const Roles& m,
                                           const Coef& C, const Rk4Param& R, int* flag, lds_double* b0, int tid) {
   using Tl = LdsTile<TX, TY, TZ>;
-  const int tx = tid % TX, ty = tile_row((tid / TX) % TY, TY), tz = tid / (TX * TY);
-  const int ltv = (tx + 3) + Tl::LX * ((ty + 3) + Tl::LY * (tz + 3));
+  int tx, ty, tz;
+  Tl::point(tid, tx, ty, tz);
   const PatchDesc d = P[r.patch];
-  const long p = (r.i0 + tx) + (long)(r.j0 + ty) * d.sy + (long)(r.k0 + tz) * d.sz;
+  bool live;
+  const BufIo io = tile_io(r.i0 + tx, r.j0 + ty, r.k0 + tz, d.shape[0] - 3, d.shape[1] - 3, d.shape[2] - 3, d.sy, d.sz,
+                           (int)d.n, live);
   const long ln = (long)NFIELD * d.n;
   gdouble* slab = (gdouble*)d.slab;
   const SlabFields in{slab + m.in * ln, d.n}, u0{slab + m.u0 * ln, d.n};
   const SlabFields acc{slab + m.acc * ln, d.n}, out{slab + m.out * ln, d.n};
   const SlabAux aux{slab + kResidualBase * d.n, d.n};
   LdsRk4<STAGE, TX, TY, TZ, SlabFields, SlabFields, SlabAux> X{
-      {in, in, C, b0, b0 + (kLdsBuffers / 2) * Tl::NPAD, p, ltv, (r.i0 - 3) + (r.j0 - 3) * d.sy + (r.k0 - 3) * d.sz,
+      {in, in, C, b0, b0 + (kLdsBuffers / 2) * Tl::NPAD, io, Tl::lds_index(tx, ty, tz, d.sz),
+       (r.i0 - 3) + (r.j0 - 3) * d.sy + (r.k0 - 3) * d.sz,
        d.sy, d.sz, (int)d.n, tid},
-      {u0, acc, out, aux, p, R.c, R.tinny, {}}};
+      {u0, acc, out, aux, io, R.c, R.tinny, {}}};
   X.prologue();
   bssn_rhs_point<GAUGE, CO, false, false>(X, X);
   X.finish();
-  if (X.bad) *flag = 1;
+  if (X.bad && live) *flag = 1;
 }
 
 // PERSIST: a grid of resident workgroups strides over the tile list.  The

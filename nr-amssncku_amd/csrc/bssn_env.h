@@ -317,6 +317,45 @@ __device__ __forceinline__ void enforce_point(double d[6], double a[6]) {
   for (int s = 0; s < 6; ++s) a[s] -= (1.0 / 3.0) * g[s] * trA;
 }
 
+// How a sink reads and writes the arrays at its point.
+// PtrIo: a plain index.
+struct PtrIo {
+  long p;
+  template <class P>
+  __device__ __forceinline__ double ld(P a) const {
+    return a[p];
+  }
+  template <class P>
+  __device__ __forceinline__ void st(P a, double x) const {
+    a[p] = x;
+  }
+};
+// BufIo: byte offsets into raw buffers of `bytes` bytes over each array (base
+// in scalar registers, one shared per-lane offset).  A lane whose store
+// offset is kDropStore (a thread of a partial tile past the interior) stores
+// nothing: the hardware drops buffer stores at or past the buffer's end, so
+// the point kernels mask their stores without a branch.  (Shared 32-bit
+// offsets also took the tile-list step of 37 patches from 22.8 to 21.8 ms.)
+constexpr unsigned kDropStore = 0xFFFFFFF8u;  // >= bytes of any array (at most 2^29 - 1 points)
+struct BufIo {
+  unsigned vo;     // byte offset of the point (clamped into the interior)
+  unsigned vs;     // vo, or kDropStore
+  unsigned bytes;  // of one array
+  template <class P>
+  __device__ __forceinline__ __amdgpu_buffer_rsrc_t rsrc(P a) const {
+    return __builtin_amdgcn_make_buffer_rsrc((void*)a, (short)0, (int)bytes, 0x00020000);
+  }
+  template <class P>
+  __device__ __forceinline__ double ld(P a) const {
+    return __builtin_bit_cast(double, __builtin_amdgcn_raw_buffer_load_b64(rsrc(a), vo, 0, 0));
+  }
+  template <class P>
+  __device__ __forceinline__ void st(P a, double x) const {
+    typedef unsigned v2u __attribute__((ext_vector_type(2)));
+    __builtin_amdgcn_raw_buffer_store_b64(__builtin_bit_cast(v2u, x), rsrc(a), vs, 0, 0);
+  }
+};
+
 // RK4 sub-step sink (rungekutta4_rout.f90:110-128 fused into the RHS
 // epilogue), followed by the lower bound on chi (fmisc.f90:1644-1657) and,
 // for sub-steps 0-2, the enforce_ga that the next RHS call applies to its
@@ -478,14 +517,14 @@ struct UpdateItems {
 // Same epilogue with the sub-step fixed at compile time: the interior kernels
 // use this form, since a runtime stage makes the compiler duplicate the whole
 // point computation per stage branch (and blows the register budget).
-template <int STAGE, class FI = FieldsIn, class FO = FieldsOut, class AX = AuxOut>
+template <int STAGE, class FI = FieldsIn, class FO = FieldsOut, class AX = AuxOut, class IO = PtrIo>
 struct Rk4SinkT {
   static constexpr int kPin = STAGE == 0 ? 1 : 2;
   const FI& U0;
   const FO& ACC;
   const FO& OUT;
   const AX& X;
-  long p;
+  IO io;
   double c, tinny;
   double gA[12];
   // U0 and ACC at p of the fields of the LDS environment's open pair of
@@ -513,8 +552,8 @@ struct Rk4SinkT {
     for (int h = 0; h < 2; ++h) {
       if ((v[h] >= GAMX && v[h] <= GAMZ) || v[h] == TRK) continue;
       nv[h] = v[h];
-      nu[h] = U0.ptr(v[h])[p];
-      na[h] = STAGE > 0 ? (double)ACC.ptr(v[h])[p] : 0.0;
+      nu[h] = io.ld(U0.ptr(v[h]));
+      na[h] = STAGE > 0 ? io.ld(ACC.ptr(v[h])) : 0.0;
     }
   }
 
@@ -526,8 +565,8 @@ struct Rk4SinkT {
     } else if (v == pv[1]) {
       u0v = pu[1], av = pa[1];
     } else {
-      u0v = U0.ptr(v)[p];
-      if (STAGE > 0) av = ACC.ptr(v)[p];
+      u0v = io.ld(U0.ptr(v));
+      if (STAGE > 0) av = io.ld(ACC.ptr(v));
     }
   }
   // rungekutta4_rout at p for field v from its rhs k: the accumulator's new
@@ -554,20 +593,20 @@ struct Rk4SinkT {
   __device__ __forceinline__ void put_loaded(int v, double k, double u0v, double av) {
     double accv, u;
     rk4_values(v, k, u0v, av, accv, u);
-    if (STAGE < 3) ACC.ptr(v)[p] = accv;
+    if (STAGE < 3) io.st(ACC.ptr(v), accv);
     if (STAGE < 3 && v >= DXX && v <= AZZ)
       gA[v - DXX] = u;
     else
-      OUT.ptr(v)[p] = u;
+      io.st(OUT.ptr(v), u);
   }
   __device__ __forceinline__ void gam(int, double) {}
   __device__ __forceinline__ void ric(int, double) {}
-  __device__ __forceinline__ void res(int a, double x) { X.resp(a)[p] = x; }
+  __device__ __forceinline__ void res(int a, double x) { io.st(X.resp(a), x); }
   __device__ __forceinline__ void finish() {
     if (STAGE < 3) {
       enforce_point(gA, gA + 6);
 #pragma unroll
-      for (int s = 0; s < 12; ++s) OUT.ptr(DXX + s)[p] = gA[s];
+      for (int s = 0; s < 12; ++s) io.st(OUT.ptr(DXX + s), gA[s]);
     }
   }
 };

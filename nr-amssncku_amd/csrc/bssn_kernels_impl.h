@@ -135,24 +135,28 @@ AMSS_POINT_KERNEL rk4_interior_kernel(FieldsIn in, FieldsIn u0, FieldsOut acc, F
   S.finish();
 }
 
-// LDS-staged variant: 8x8xTZ-point tiles (TZ = 8 where the box holds whole
-// 8-deep tiles, else 4), halo tiles of every field group in LDS
-// (double-buffered, filled by direct global->LDS loads).  A 1-D grid of
+// LDS-staged variant: 8x8xTZ-point tiles, halo tiles of every field group in
+// LDS (double-buffered, filled by direct global->LDS loads).  A 1-D grid of
 // tiles in XCD-contiguous order: consecutive tiles, whose halos overlap, run
-// behind the same L2.  The 8-deep tile (512 threads, one workgroup per CU)
-// re-reads 14/8 instead of 10/4 z-planes of halo per interior plane.
+// behind the same L2.  The tiles cover the box whole: threads of a partial
+// tile past it compute on a clamped point and store nothing (remainder slabs
+// on the direct kernel took 120-155 us each and sub-step, whatever their size:
+// a coarse step of a 64^3 patch and a nested one of 76^3 with them 10.2 ms,
+// with partial tiles 7.4 ms).  The 8-deep tile
+// (512 threads, one workgroup per CU) re-reads 14/8 instead of 10/4 z-planes
+// of halo per interior plane.  Instantiated in bssn_lds_g<G>[_odd].hip.
 constexpr int kLdsTX = 8, kLdsTY = 8, kLdsTZ = 4;
 #ifndef AMSS_LDS_WAVES
 #define AMSS_LDS_WAVES 2
 #endif
-template <int GAUGE, int STAGE, bool CO, int TZ>
+template <int GAUGE, int STAGE, bool CO, int TZ, bool ODD>
 __global__ void __launch_bounds__(kLdsTX * kLdsTY * TZ) __attribute__((amdgpu_waves_per_eu(AMSS_LDS_WAVES, AMSS_LDS_WAVES)))
 rk4_lds_kernel(FieldsIn in, FieldsIn u0, FieldsOut acc, FieldsOut out, AuxOut aux, Box box,
                                  Coef C, Rk4Param R, int* flag, long nfill) {
-  using Tl = LdsTile<kLdsTX, kLdsTY, TZ>;
+  using Tl = LdsTile<kLdsTX, kLdsTY, TZ, ODD>;
   __shared__ __attribute__((aligned(16))) double tiles[kLdsBuffers * Tl::NPAD];
-  const int gx = (box.hi[0] - box.lo[0]) / kLdsTX, gy = (box.hi[1] - box.lo[1]) / kLdsTY;
-  const int ntiles = gx * gy * ((box.hi[2] - box.lo[2]) / TZ);
+  const int gx = (box.hi[0] - box.lo[0] + kLdsTX - 1) / kLdsTX, gy = (box.hi[1] - box.lo[1] + kLdsTY - 1) / kLdsTY;
+  const int ntiles = gx * gy * ((box.hi[2] - box.lo[2] + TZ - 1) / TZ);
   if ((int)blockIdx.x >= ntiles) {
     // the frozen-ghost fill of the nfill points outside [3, n - 3) of the
     // array (nfill is 0 when the caller fills them), in the workgroups after
@@ -168,24 +172,23 @@ rk4_lds_kernel(FieldsIn in, FieldsIn u0, FieldsOut acc, FieldsOut out, AuxOut au
     }
     return;
   }
-  const int tx = threadIdx.x % kLdsTX, ty = tile_row((threadIdx.x / kLdsTX) % kLdsTY, kLdsTY),
-            tz = threadIdx.x / (kLdsTX * kLdsTY);
+  int tx, ty, tz;
+  Tl::point((int)threadIdx.x, tx, ty, tz);
   const int b = xcd_spread(blockIdx.x, ntiles);
   const int i0 = box.lo[0] + (b % gx) * kLdsTX, j0 = box.lo[1] + ((b / gx) % gy) * kLdsTY;
   const int k0 = box.lo[2] + (b / (gx * gy)) * TZ;
-  const int i = i0 + tx, j = j0 + ty, k = k0 + tz;
-  // the launch covers whole tiles only (remainder slabs go to the direct kernel)
-  const long p = i + j * box.sy + k * box.sz;
   const int N = box.n[0] * box.n[1] * box.n[2];
+  bool live;
+  const BufIo io = tile_io(i0 + tx, j0 + ty, k0 + tz, box.hi[0], box.hi[1], box.hi[2], (int)box.sy, (int)box.sz, N, live);
   lds_double* t0 = (lds_double*)tiles;
-  LdsRk4<STAGE, kLdsTX, kLdsTY, TZ, FieldsIn, FieldsOut, AuxOut, true> X{
-      {in, in, C, t0, t0 + (kLdsBuffers / 2) * Tl::NPAD, p, (tx + 3) + Tl::LX * ((ty + 3) + Tl::LY * (tz + 3)),
-       (int)((i0 - 3) + (j0 - 3) * box.sy + (k0 - 3) * box.sz), (int)box.sy, (int)box.sz, N, (int)threadIdx.x},
-      {u0, acc, out, aux, p, R.c, R.tinny, {}}};
+  LdsRk4<STAGE, kLdsTX, kLdsTY, TZ, FieldsIn, FieldsOut, AuxOut, true, ODD> X{
+      {in, in, C, t0, t0 + (kLdsBuffers / 2) * Tl::NPAD, io, Tl::lds_index(tx, ty, tz, (int)box.sz),
+       (int)((i0 - 3) + (j0 - 3) * box.sy + (k0 - 3) * box.sz), (int)box.sy, (int)box.sz, N, (int)threadIdx.x, tz + 3},
+      {u0, acc, out, aux, io, R.c, R.tinny, {}}};
   X.prologue();
   bssn_rhs_point<GAUGE, CO, false, false>(X, X);
   X.finish();
-  if (X.bad) *flag = 1;
+  if (X.bad && live) *flag = 1;
 }
 
 // sg: the Sommerfeld faces of the array (none when sg.faces == 0).  The
@@ -295,52 +298,21 @@ void launch_rhs_gauge(const FieldsIn& in, const FieldsIn& mat, const FieldsOut& 
 #undef AMSS_REDGE
 }
 
+// The fused sub-step of an interior box on LDS tiles (ODD: an odd row pitch).
+template <int G, bool ODD>
+void launch_rk4_lds(const FieldsIn& in, const FieldsIn& u0, const FieldsOut& acc, const FieldsOut& out,
+                    const AuxOut& aux, const Box& box, const Coef& C, const Rk4Param& R, bool want_res, int* flag,
+                    hipStream_t s);
+
 template <int G>
 void launch_rk4_gauge(const FieldsIn& in, const FieldsIn& u0, const FieldsOut& acc, const FieldsOut& out,
                       const AuxOut& aux, const Box& box, const Coef& C, const Rk4Param& R, bool want_res, int* flag,
                       bool edge, hipStream_t s, bool interior, const SommerGeom& sg) {
-  // The LDS kernel's 16-byte direct loads start at even x of a row, which is
-  // 16-byte aligned only when the row pitch is even; odd pitches go direct.
-  if (interior && !box_empty(box) && R.variant == 1 && (box.sy % 2) == 0) {
-    // LDS kernel on the largest tile-aligned sub-box, the direct kernel on the rest
-    Box core = box;
-    const int tz = box.hi[2] - box.lo[2] >= 8 ? 8 : kLdsTZ;
-    const int T[3] = {kLdsTX, kLdsTY, tz};
-    for (int a = 0; a < 3; ++a) core.hi[a] = box.lo[a] + (box.hi[a] - box.lo[a]) / T[a] * T[a];
-    if (!box_empty(core)) {
-      const unsigned ntile = (unsigned)((core.hi[0] - core.lo[0]) / kLdsTX) * ((core.hi[1] - core.lo[1]) / kLdsTY) *
-                             ((core.hi[2] - core.lo[2]) / tz);
-      const int nt = kLdsTX * kLdsTY * tz;
-      // the fused frozen-ghost fill (none unless rk4_fuses_fill)
-      const long nfill = rk4_fuses_fill(box, R) ? ghost3_count(box.n[0], box.n[1], box.n[2]) : 0;
-      const unsigned gr = ntile + (unsigned)((nfill + nt - 1) / nt);
-#define AMSS_LDS(TZ)                                                                                          \
-  switch (R.stage) {                                                                                          \
-    case 0:                                                                                                   \
-      if (want_res) rk4_lds_kernel<G, 0, true, TZ><<<gr, nt, 0, s>>>(in, u0, acc, out, aux, core, C, R, flag, nfill); \
-      else rk4_lds_kernel<G, 0, false, TZ><<<gr, nt, 0, s>>>(in, u0, acc, out, aux, core, C, R, flag, nfill);         \
-      break;                                                                                                  \
-    case 1: rk4_lds_kernel<G, 1, false, TZ><<<gr, nt, 0, s>>>(in, u0, acc, out, aux, core, C, R, flag, nfill); break; \
-    case 2: rk4_lds_kernel<G, 2, false, TZ><<<gr, nt, 0, s>>>(in, u0, acc, out, aux, core, C, R, flag, nfill); break; \
-    default: rk4_lds_kernel<G, 3, false, TZ><<<gr, nt, 0, s>>>(in, u0, acc, out, aux, core, C, R, flag, nfill); break; \
-  }
-      if (tz == 8) {
-        AMSS_LDS(8)
-      } else {
-        AMSS_LDS(4)
-      }
-#undef AMSS_LDS
-    }
-    Rk4Param Rd = R;
-    Rd.variant = 0;
-    for (int a = 0; a < 3; ++a) {  // remainder slab [core.hi[a], box.hi[a]) along axis a
-      Box rem = box;
-      for (int c = 0; c < a; ++c) rem.hi[c] = core.hi[c];
-      rem.lo[a] = core.hi[a];
-      if (!box_empty(rem)) launch_rk4_gauge<G>(in, u0, acc, out, aux, rem, C, Rd, want_res, flag, false, s, true, sg);
-    }
+  if (interior && !box_empty(box) && R.variant == 1) {
+    if (box.sy % 2 == 0) launch_rk4_lds<G, false>(in, u0, acc, out, aux, box, C, R, want_res, flag, s);
+    else launch_rk4_lds<G, true>(in, u0, acc, out, aux, box, C, R, want_res, flag, s);
   } else if (interior && !box_empty(box)) {
-    const dim3 gr = interior_grid(box);  // also variant 1 on an odd row pitch
+    const dim3 gr = interior_grid(box);
     switch (R.stage) {
       case 0:
         if (want_res) rk4_interior_kernel<G, 0, true><<<gr, kRhsThreads, 0, s>>>(in, u0, acc, out, aux, box, C, R, flag);

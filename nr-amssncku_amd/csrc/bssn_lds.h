@@ -1,7 +1,8 @@
 // bssn_lds.h -- LDS-staged stencil environment for the fused RHS kernels.
 //
-// A 256-thread workgroup owns a TX x TY x TZ tile of interior points (one
-// point per thread).  For every field group of the algebra the tile plus a
+// A workgroup owns a TX x TY x TZ tile of interior points (one point per
+// thread; the threads of a partial tile past the interior compute on clamped
+// points and store nothing).  For every field group of the algebra the tile plus a
 // 3-point halo of that field, (TX+6)(TY+6)(TZ+6) doubles, sits in LDS; every
 // stencil of the group (gradient, Hessian incl. mixed, upwind, KO) reads it
 // from there with compile-time offsets.  Two tile buffers alternate: while
@@ -38,27 +39,64 @@ __host__ __device__ constexpr int group_extra(int v) {
 // every stencil offset a 64-bit flat address).
 typedef __attribute__((address_space(3))) double lds_double;
 
-#ifndef AMSS_ROWPERM
-#define AMSS_ROWPERM 1
-#endif
 // Tile row of a thread's row index r (of TY): with 8 rows a 16-lane LDS
 // access group can hold rows y and y + 4, whose 14-double pitch puts them
 // 112 dwords apart (16 mod 32 banks).
-__host__ __device__ constexpr int tile_row(int r, int TY) {
-  return (AMSS_ROWPERM && TY == 8) ? ((r & 1) ? 4 + (r >> 1) : (r >> 1)) : r;
-}
+__host__ __device__ constexpr int tile_row(int r, int TY) { return TY == 8 ? ((r & 1) ? 4 + (r >> 1) : (r >> 1)) : r; }
 
-template <int TX, int TY, int TZ>
+// The LDS layout of one field's halo tile.  The direct loads move 16-byte
+// aligned chunks, so an element's LDS index and its index in the array (plus
+// the array's own offset from 16 bytes, LdsEnv::odd_base) must have the same
+// parity throughout the tile.
+//  EVEN row pitch of the arrays: rows of TX + 6 doubles, planes without gaps
+//    (rows start at an even x, and so does every chunk).
+//  ODD pitch: rows of 15 doubles (elements x = -1 .. 13; -1 is padding whose
+//    chunk may hold it and x = 0), planes of 216 (16 banks apart, so that a
+//    wave of 8 x 4 x 2 points has each 16-lane access group -- 8 points of x
+//    on two planes -- on disjoint banks); where the arrays' plane pitch is odd
+//    too, odd planes start one double later.  A sub-step of 85^3 points takes
+//    395 us (the direct kernel, which took odd pitches before, about 650); the
+//    same tiles filled by 4-byte loads spilled scalar registers (730 us with
+//    the residuals).
+template <int TX, int TY, int TZ, bool ODD = false>
 struct LdsTile {
   static constexpr int LX = TX + 6, LY = TY + 6, LZ = TZ + 6;
-  static constexpr int NE = LX * LY * LZ;  // doubles per field tile
-  static constexpr int NCH = NE / 2;       // 16-byte chunks
+  static constexpr int PY = ODD ? LX + 1 : LX, PZ = ODD ? 216 : LX * LY;  // LDS pitches
+  static constexpr int NCH = PZ * LZ / 2;  // 16-byte chunks
   static constexpr int NT = TX * TY * TZ;  // threads
   static constexpr int ROUNDS = (NCH + NT - 1) / NT;
   static constexpr int NPAD = 2 * ROUNDS * NT;  // doubles per buffer: whole rounds, no bounds branches
   static_assert(LX % 2 == 0, "tile rows must hold whole 16-byte chunks");
   static_assert(NT % 64 == 0, "whole waves");
+  static_assert(!ODD || (TX == 8 && TY == 8 && PY * LY + 2 <= PZ), "odd pitch: 8 x 8 rows");
+  static_assert(PZ * LZ < NPAD || !ODD, "room for the last plane's shift");
+
+  // the tile point of thread tid
+  __device__ __forceinline__ static void point(int tid, int& tx, int& ty, int& tz) {
+    if (ODD) {
+      tx = tid & 7;
+      ty = ((tid >> 4) & 3) + 4 * ((tid >> 6) & 1);
+      tz = ((tid >> 3) & 1) + 2 * (tid >> 7);
+    } else {
+      tx = tid % TX;
+      ty = tile_row((tid / TX) % TY, TY);
+      tz = tid / (TX * TY);
+    }
+  }
+  // its LDS index (ODD: sz is the arrays' plane pitch)
+  __device__ __forceinline__ static int lds_index(int tx, int ty, int tz, int sz) {
+    return (tx + 3) + PY * (ty + 3) + PZ * (tz + 3) + (ODD ? (sz & 1 & (tz + 3)) : 0);
+  }
 };
+
+// Array access of the tile point (i, j, k): live inside the interior [.., hi),
+// else clamped into it and storing nothing.
+__device__ __forceinline__ BufIo tile_io(int i, int j, int k, int hx, int hy, int hz, int sy, int sz, int n,
+                                         bool& live) {
+  live = i < hx && j < hy && k < hz;
+  const unsigned vo = (unsigned)(min(i, hx - 1) + min(j, hy - 1) * sy + min(k, hz - 1) * sz) * 8u;
+  return BufIo{vo, live ? vo : kDropStore, (unsigned)n * 8u};
+}
 
 #ifndef AMSS_LDS_FENCE
 #define AMSS_LDS_FENCE 1
@@ -78,48 +116,67 @@ constexpr int kLdsBuffers = AMSS_LDS_PAIRS ? 4 : 2;
 #endif
 // Self: a type deriving from this environment and from the RK4 epilogue,
 // whose prefetch(v0, v1) the environment calls for each pair (void: none).
-template <int TX, int TY, int TZ, class FI = FieldsIn, class Self = void>
+template <int TX, int TY, int TZ, class FI = FieldsIn, class Self = void, bool ODD = false>
 struct LdsEnv {
   static constexpr bool kFence = AMSS_LDS_FENCE;
-  using T = LdsTile<TX, TY, TZ>;
-  static constexpr long SY = T::LX, SZ = (long)T::LX * T::LY;
+  using T = LdsTile<TX, TY, TZ, ODD>;
+  static constexpr long SY = T::PY, SZ = T::PZ;
 
   const FI& F;
   const FI& M;
   const Coef& C;
   lds_double* buf0;   // two pairs of LDS tile buffers (2 x NPAD doubles each)
   lds_double* buf1;
-  long p;         // global index of this thread's point (clamped into the array)
+  BufIo at_p;     // this thread's point (clamped into the interior) in the arrays
   int lt;         // LDS index of this thread's point
   int gbase;      // global index of tile element (0,0,0)
   int sy, sz;     // global strides
   int gmax;       // number of points of one field
   int tid;        // thread index in the workgroup
+  int plane = 0;  // ODD: the point's plane in the tile, halo included
+  // ODD: LDS indices of the point in the open group's tile, and the base of
+  // reads an odd number of planes away (the odd planes' shift)
+  int ltc = 0, ltz = 0;
   int g = 0;      // next group to open
   bool bad = false;  // a NaN among the centre values of the first 21 fields (bssn_rhs.f90:110-113)
   double top[NFIELD];  // centre values the algebra reads before its first group (in_top)
   int xf[2] = {-1, -1}, nxf[2] = {-1, -1};  // group_extra of the open (next) pair's fields
   double xv[2], nxv[2];                      // ... and their centre values, loaded a pair ahead
 
-  // Stream the halo tile of field v into buffer b: every lane issues ROUNDS
-  // 16-byte direct global->LDS loads.  The buffer is padded to whole rounds,
-  // so chunks past the tile land in the padding (reading a clamped, valid
-  // address) and the loop has no bounds branches -- branches here split the
-  // point kernel into many blocks and wreck its register allocation.
+  // Stream the halo tile of field v into buffer b by direct global->LDS
+  // loads.  The buffer is padded to whole rounds, so chunks past the tile
+  // land in the padding and the loop has no bounds branches -- branches here
+  // split the point kernel into many blocks and wreck its register
+  // allocation.  Addresses outside the array (the front and end corners, and
+  // the part of a partial tile past the interior's halo, which no live point
+  // reads) are clamped to valid ones.
   __device__ __forceinline__ void issue(int v, lds_double* b) const {
     const auto base = F.ptr(v);
     const int wave = tid >> 6;
+    const int ob = odd_base(v);
 #pragma unroll
     for (int r = 0; r < T::ROUNDS; ++r) {
       const int c = r * T::NT + tid;
       const int e = 2 * c;
-      const int x = e % T::LX, y = (e / T::LX) % T::LY, z = e / (T::LX * T::LY);
-      int gi = gbase + x + y * sy + z * sz;  // < 2^29 points per field
-      gi = gi < 0 ? 0 : (gi > gmax - 2 ? gmax - 2 : gi);
+      int gi;
+      if constexpr (ODD) {
+        const int z = e / T::PZ, t = e - z * T::PZ + 1 - (sz & 1 & z) - ob, y = t / T::PY, x = t - y * T::PY - 1;
+        gi = gbase + x + y * sy + z * sz;  // of e's parity: a clamped index keeps it
+        gi = min(max(gi, gi & 1), gmax - 2 - ((gi ^ gmax) & 1));
+      } else {
+        const int x = e % T::LX, y = (e / T::LX) % T::LY, z = e / (T::LX * T::LY);
+        gi = gbase + x + y * sy + z * sz;  // < 2^29 points per field
+        gi = min(max(gi, 0), gmax - 2);
+      }
       __builtin_amdgcn_global_load_lds((__attribute__((address_space(1))) void*)(base + gi),
                                        (__attribute__((address_space(3))) void*)(b + 2 * (r * T::NT + wave * 64)),
                                        16, 0, 0);
     }
+  }
+  // ODD: 1 where the tile's first element lies on the second half of a
+  // 16-byte chunk of field v; its LDS image then starts at index 1.
+  __device__ __forceinline__ int odd_base(int v) const {
+    return ODD ? (int)(((uintptr_t)F.ptr(v) >> 3) + (unsigned)gbase) & 1 : 0;
   }
   // Groups are staged two at a time: groups 2q and 2q+1 share pair q & 1,
   // so a tile needs one barrier per two field groups.
@@ -135,7 +192,7 @@ struct LdsEnv {
 #pragma unroll
     for (int h = 0; h < 2; ++h) {
       nxf[h] = group_extra(group_field(g0 + h));
-      if (nxf[h] >= 0) nxv[h] = F.ptr(nxf[h])[p];
+      if (nxf[h] >= 0) nxv[h] = at_p.ld(F.ptr(nxf[h]));
     }
     if constexpr (!std::is_void_v<Self>) static_cast<Self*>(this)->prefetch(group_field(g0), group_field(g0 + 1));
   }
@@ -157,7 +214,7 @@ struct LdsEnv {
     if (AMSS_TOP) {
 #pragma unroll
       for (int v = 0; v < NFIELD; ++v)
-        if (in_top(v)) top[v] = F.ptr(v)[p];
+        if (in_top(v)) top[v] = at_p.ld(F.ptr(v));
     }
     if (AMSS_LDS_PAIRS) ahead(0);
     __builtin_amdgcn_sched_barrier(0);
@@ -188,24 +245,35 @@ struct LdsEnv {
     }
     if constexpr (!std::is_void_v<Self>) static_cast<Self*>(this)->sink_flush();
     ++g;
+    if constexpr (ODD) {
+      ltc = lt + odd_base(v);
+      ltz = ltc + (sz & 1) - 2 * (sz & 1 & plane);
+    }
     if (v < 21) {
-      const double x = cur()[lt];
+      const double x = at(v, 0);
       bad |= !(x == x);
     }
   }
   __device__ __forceinline__ void end() const {}
 
-  __device__ __forceinline__ double at(int, long o) const { return cur()[lt + o]; }
+  __device__ __forceinline__ double at(int, long o) const {
+    if constexpr (ODD) {
+      const long dz = (o + 4 * SZ + SZ / 2) / SZ - 4;  // a constant, as o is
+      return cur()[((dz & 1) ? ltz : ltc) + o];
+    } else {
+      return cur()[lt + o];
+    }
+  }
   // the centre value of the open group's field is in its halo tile; the
   // pair's extra centre values were loaded at its barrier
   __device__ __forceinline__ double val(int v) const {
     if (AMSS_TOP && g == 0 && in_top(v)) return top[v];
-    if (g > 0 && v == group_field(g - 1)) return cur()[lt];
+    if (g > 0 && v == group_field(g - 1)) return at(v, 0);
     if (v == xf[0]) return xv[0];
     if (v == xf[1]) return xv[1];
-    return F.ptr(v)[p];
+    return at_p.ld(F.ptr(v));
   }
-  __device__ __forceinline__ double mat(int m) const { return M.ptr(m)[p]; }
+  __device__ __forceinline__ double mat(int m) const { return at_p.ld(M.ptr(m)); }
 
   __device__ __forceinline__ double d1(int v, long s) const {
     return (at(v, -2 * s) - at(v, 2 * s)) + 8.0 * (at(v, s) - at(v, -s));
@@ -270,9 +338,10 @@ struct LdsEnv {
 // kernel +0.9%, the tile-list kernel -1.4%, so only the former defers; and
 // sub-step 3, one store per field, gains nothing.
 template <int STAGE, int TX, int TY, int TZ, class FI = FieldsIn, class FO = FieldsOut, class AX = AuxOut,
-          bool DEFER = false>
-struct LdsRk4 : LdsEnv<TX, TY, TZ, FI, LdsRk4<STAGE, TX, TY, TZ, FI, FO, AX, DEFER>>, Rk4SinkT<STAGE, FI, FO, AX> {
-  using Sink = Rk4SinkT<STAGE, FI, FO, AX>;
+          bool DEFER = false, bool ODD = false>
+struct LdsRk4 : LdsEnv<TX, TY, TZ, FI, LdsRk4<STAGE, TX, TY, TZ, FI, FO, AX, DEFER, ODD>, ODD>,
+                Rk4SinkT<STAGE, FI, FO, AX, BufIo> {
+  using Sink = Rk4SinkT<STAGE, FI, FO, AX, BufIo>;
   static constexpr bool kDefer = DEFER && STAGE < 3;
   int dv = -1;
   double dacc, dout;
@@ -280,8 +349,8 @@ struct LdsRk4 : LdsEnv<TX, TY, TZ, FI, LdsRk4<STAGE, TX, TY, TZ, FI, FO, AX, DEF
   __device__ __forceinline__ void prefetch(int v0, int v1) { Sink::prefetch(v0, v1); }
   __device__ __forceinline__ void sink_flush() {
     if (!kDefer || dv < 0) return;
-    if (STAGE < 3) Sink::ACC.ptr(dv)[Sink::p] = dacc;
-    if (!(STAGE < 3 && dv >= DXX && dv <= AZZ)) Sink::OUT.ptr(dv)[Sink::p] = dout;
+    if (STAGE < 3) Sink::io.st(Sink::ACC.ptr(dv), dacc);
+    if (!(STAGE < 3 && dv >= DXX && dv <= AZZ)) Sink::io.st(Sink::OUT.ptr(dv), dout);
     dv = -1;
   }
   __device__ __forceinline__ void put(int v, double k) {

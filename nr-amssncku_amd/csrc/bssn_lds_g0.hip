@@ -1,0 +1,10 @@
+// The LDS-staged fused sub-step for GAUGE 0, even row pitches.
+#include "bssn_lds_launch.h"
+
+namespace amss {
+
+template void launch_rk4_lds<0, false>(const FieldsIn&, const FieldsIn&, const FieldsOut&, const FieldsOut&,
+                                        const AuxOut&, const Box&, const Coef&, const Rk4Param&, bool, int*,
+                                        hipStream_t);
+
+}  // namespace amss
