@@ -24,11 +24,11 @@
 
 namespace amss {
 
-template <int ORD, int NRM>
-struct EdgeLdsEnv : EdgeStencils<ORD, EdgeLdsEnv<ORD, NRM>> {
+template <int ORD, int NRM, bool ODD, bool MIRROR>
+struct EdgeLdsEnv : EdgeStencils<ORD, EdgeLdsEnv<ORD, NRM, ODD, MIRROR>, MIRROR> {
   static constexpr bool kFence = true;
-  using Base = EdgeStencils<ORD, EdgeLdsEnv<ORD, NRM>>;
-  using W = EdgeWindow<NRM>;
+  using Base = EdgeStencils<ORD, EdgeLdsEnv<ORD, NRM, ODD, MIRROR>, MIRROR>;
+  using W = EdgeWindow<NRM, ODD>;
   const FieldsIn& F;
   const FieldsIn& M;
   lds_double* buf;  // two window buffers of W::PAD doubles
@@ -38,7 +38,11 @@ struct EdgeLdsEnv : EdgeStencils<ORD, EdgeLdsEnv<ORD, NRM>> {
   int tid;
   int wlo[3];       // array index of window element (0, 0, 0)
   int mir;          // bit a: the window reaches below index 0 on a symmetry plane of axis a
-  int lt;           // LDS index of the point
+  int lt;           // LDS index of the point (ODD: with the window at 0)
+  int pz;           // its plane in the window
+  // ODD: LDS indices of the point in the open group's window, and the base of
+  // reads an odd number of planes away (the odd planes' shift)
+  int ltc = 0, ltz = 0;
   // stencil reads address one base, the point's lowest neighbour (-3, -3,
   // -3), so every offset is a non-negative immediate, in both buffers
   static constexpr int kLow = 3 + 3 * W::P0 + 3 * W::P01;
@@ -61,7 +65,8 @@ struct EdgeLdsEnv : EdgeStencils<ORD, EdgeLdsEnv<ORD, NRM>> {
       if (box.mlo[a] < 0 && wlo[a] < 0) mir |= 1 << a;
     }
     gbase = wlo[0] + wlo[1] * sy + wlo[2] * sz;
-    lt = (q[0] - wlo[0]) + (q[1] - wlo[1]) * W::P0 + (q[2] - wlo[2]) * W::P01;
+    pz = q[2] - wlo[2];
+    lt = W::index(q[0] - wlo[0], q[1] - wlo[1], pz, sz, 0);
   }
 
   // Stream field v's window into buffer b: ROUNDS 16-byte direct loads per
@@ -71,16 +76,21 @@ struct EdgeLdsEnv : EdgeStencils<ORD, EdgeLdsEnv<ORD, NRM>> {
   __device__ __forceinline__ void issue(int v, lds_double* b) const {
     const auto base = F.ptr(v);
     const int wave = tid >> 6;
+    const int ob = odd_base(v);
 #pragma unroll
     for (int r = 0; r < W::ROUNDS; ++r) {
-      const int e = 2 * (r * kEdgeThreads + tid);
-      const int x = e % W::P0, y = (e / W::P0) % W::W1, z = e / W::P01;
-      int gi = gbase + x + y * sy + z * sz;
-      gi = gi < 0 ? 0 : (gi > gmax - 2 ? gmax - 2 : gi);
+      int x, y, z;
+      W::element(2 * (r * kEdgeThreads + tid), sz, ob, x, y, z);
+      const int gi = W::clamp(gbase + x + y * sy + z * sz, gmax);
       __builtin_amdgcn_global_load_lds((__attribute__((address_space(1))) void*)(base + gi),
                                        (__attribute__((address_space(3))) void*)(b + 2 * (r * kEdgeThreads + wave * 64)),
                                        16, 0, 0);
     }
+  }
+  // ODD: 1 where the window's first element lies on the second half of a
+  // 16-byte chunk of field v; its LDS image then starts at index 1.
+  __device__ __forceinline__ int odd_base(int v) const {
+    return ODD ? (int)(((uintptr_t)F.ptr(v) >> 3) + (unsigned)gbase) & 1 : 0;
   }
   // Below a symmetry plane the window holds the mirror image of the field
   // with its parity (symmetry_bd, fmisc.f90:877-901): index -m-1 of axis a
@@ -88,23 +98,22 @@ struct EdgeLdsEnv : EdgeStencils<ORD, EdgeLdsEnv<ORD, NRM>> {
   // cells read only cells at or above 0 on the mirrored axes, which this
   // pass does not write.
   __device__ __forceinline__ void mirror(int v, lds_double* b) const {
-    for (int c = tid; c < W::NE; c += kEdgeThreads) {
-      const int x[3] = {c % W::P0, (c / W::P0) % W::W1, c / W::P01};
-      int src = 0;
+    const int ob = odd_base(v);
+    for (int c = tid; c < W::W0 * W::W1 * W::W2; c += kEdgeThreads) {
+      const int x[3] = {c % W::W0, (c / W::W0) % W::W1, c / (W::W0 * W::W1)};
+      int m[3];
       double s = 1.0;
       bool img = false;
-      const int pitch[3] = {1, W::P0, W::P01};
 #pragma unroll
       for (int a = 0; a < 3; ++a) {
-        int m = wlo[a] + x[a];
-        if (((mir >> a) & 1) && m < 0) {
-          m = -m - 1;
+        m[a] = wlo[a] + x[a];
+        if (((mir >> a) & 1) && m[a] < 0) {
+          m[a] = -m[a] - 1;
           s *= parity(v, a);
           img = true;
         }
-        src += (m - wlo[a]) * pitch[a];
       }
-      if (img) b[c] = s * b[src];
+      if (img) b[W::index(x[0], x[1], x[2], sz, ob)] = s * b[W::index(m[0] - wlo[0], m[1] - wlo[1], m[2] - wlo[2], sz, ob)];
     }
   }
   __device__ __forceinline__ lds_double* slot(int grp) const { return buf + (grp & 1) * W::PAD; }
@@ -128,21 +137,26 @@ struct EdgeLdsEnv : EdgeStencils<ORD, EdgeLdsEnv<ORD, NRM>> {
     __builtin_amdgcn_s_waitcnt(0);
     __syncthreads();
     if (g + 1 < NFIELD) issue(group_field(g + 1), slot(g + 1));
-    if (mir) {
+    if (MIRROR && mir) {
       mirror(v, slot(g));
       __syncthreads();
     }
     ++g;
-    if (v < 21 && live) {
-      const double x = cur()[lt];
-      bad |= !(x == x);
+    if constexpr (ODD) {
+      ltc = lt + odd_base(v);
+      ltz = ltc + (sz & 1) - 2 * (sz & 1 & pz);
+    }
+    if (v < 21) {
+      const double x = rel(v, 0, 0, 0, 0.0);
+      bad |= live && !(x == x);
     }
   }
   __device__ __forceinline__ void end() const {}
 
   // every neighbour the stencils read lies in the window (mirror cells included)
   __device__ __forceinline__ double rel(int, int di, int dj, int dk, double off) const {
-    return (cur() + (lt - kLow))[kLow + di + dj * W::P0 + dk * W::P01] + off;
+    const int b = ODD ? ((dk & 1) ? ltz : ltc) : lt;
+    return (cur() + (b - kLow))[kLow + di + dj * W::P0 + dk * W::P01] + off;
   }
   // the window holds +-3 points on every side of the tile, array or not
   __device__ __forceinline__ double rel_clamped(int v, int di, int dj, int dk, double off) const {
@@ -150,7 +164,7 @@ struct EdgeLdsEnv : EdgeStencils<ORD, EdgeLdsEnv<ORD, NRM>> {
   }
   __device__ __forceinline__ double val(int v) const {
     if (g == 0 && in_top(v)) return top[v];
-    if (g > 0 && v == group_field(g - 1)) return cur()[lt];
+    if (g > 0 && v == group_field(g - 1)) return rel(v, 0, 0, 0, 0.0);
     return F.ptr(v)[p];
   }
   __device__ __forceinline__ double mat(int m) const { return M.ptr(m)[p]; }
@@ -177,14 +191,16 @@ struct CompactSink {
 #define AMSS_EDGE_LDS_WAVES 2
 #endif
 // LDS per workgroup: two window buffers of the largest window.
-constexpr int kEdgeLdsDoubles = 2 * (EdgeWindow<0>::PAD > EdgeWindow<1>::PAD
-                                         ? (EdgeWindow<0>::PAD > EdgeWindow<2>::PAD ? EdgeWindow<0>::PAD : EdgeWindow<2>::PAD)
-                                         : (EdgeWindow<1>::PAD > EdgeWindow<2>::PAD ? EdgeWindow<1>::PAD : EdgeWindow<2>::PAD));
+template <bool ODD>
+constexpr int edge_lds_doubles() {
+  constexpr int p0 = EdgeWindow<0, ODD>::PAD, p1 = EdgeWindow<1, ODD>::PAD, p2 = EdgeWindow<2, ODD>::PAD;
+  return 2 * (p0 > p1 ? (p0 > p2 ? p0 : p2) : (p1 > p2 ? p1 : p2));
+}
 
 // The right-hand side on tile lb of a shell of stencil order ORD (1 or 2,
 // whose points lie on no Sommerfeld or copy face: those are outermost-layer
 // points) whose slabs have normal axis NRM; k: the tile's compact slots.
-template <int GAUGE, bool CO, int ORD, int NRM>
+template <int GAUGE, bool CO, int ORD, int NRM, bool ODD, bool MIRROR>
 __device__ __forceinline__ void edge_rhs_tile(const FieldsIn& in, const AuxOut& aux, const Box& box,
                                               const EdgeTiles& T, int lb, const Coef& C, double* k, int* flag,
                                               lds_double* win) {
@@ -192,7 +208,7 @@ __device__ __forceinline__ void edge_rhs_tile(const FieldsIn& in, const AuxOut& 
   int q[3];
   bool live;
   edge_tile_point(t, (int)threadIdx.x, q, live);
-  EdgeLdsEnv<ORD, NRM> E(in, in, C, q, box, t, win, (int)threadIdx.x, live);
+  EdgeLdsEnv<ORD, NRM, ODD, MIRROR> E(in, in, C, q, box, t, win, (int)threadIdx.x, live);
   CompactSink S{k, aux, E.p, (int)threadIdx.x, live};
   E.prologue();
   bssn_rhs_point<GAUGE, CO, false, false>(E, S);
@@ -204,20 +220,27 @@ __device__ __forceinline__ void edge_rhs_tile(const FieldsIn& in, const AuxOut& 
 // stencil order and window layout the code is compiled for, so all tiles
 // progress together (each tile's time is a chain of one field-group load
 // and barrier after another; separate launches would queue these chains).
-template <int GAUGE, bool CO>
+// Bound by those chains and by VALU issue.  MIRROR is a variant of its own
+// because the mirror pass and the dissipation's branch cut the point
+// computation into blocks, and its registers spill: 1,020 bytes of scratch per
+// lane with them, 360 without; all tiles of a 134^3 patch 503 -> 442 us beside
+// the interior, of 70^3 and 76^3 patches 208 -> 183.  An odd-pitched patch took
+// the direct kernel before: a step of 85 x 61 x 45 interior points with the
+// copy boundary 2.74 -> 1.52 ms.
+template <int GAUGE, bool CO, bool ODD, bool MIRROR>
 __global__ void __launch_bounds__(kEdgeThreads) __attribute__((amdgpu_waves_per_eu(AMSS_EDGE_LDS_WAVES, AMSS_EDGE_LDS_WAVES)))
 rhs_edge_lds_kernel(FieldsIn in, AuxOut aux, Box box, EdgeTileSet T, Coef C, double* K, int* flag) {
-  __shared__ __attribute__((aligned(16))) double win[kEdgeLdsDoubles];
+  __shared__ __attribute__((aligned(16))) double win[edge_lds_doubles<ODD>()];
   const int b = (int)blockIdx.x, s = T.set_of(b), lb = b - T.first[s];
   double* k = K + (long)b * NFIELD * kEdgeThreads;
   lds_double* w = (lds_double*)win;
   switch (s) {
-    case 0: edge_rhs_tile<GAUGE, CO, 1, 0>(in, aux, box, T.t[0], lb, C, k, flag, w); break;
-    case 1: edge_rhs_tile<GAUGE, CO, 1, 1>(in, aux, box, T.t[1], lb, C, k, flag, w); break;
-    case 2: edge_rhs_tile<GAUGE, CO, 1, 2>(in, aux, box, T.t[2], lb, C, k, flag, w); break;
-    case 3: edge_rhs_tile<GAUGE, CO, 2, 0>(in, aux, box, T.t[3], lb, C, k, flag, w); break;
-    case 4: edge_rhs_tile<GAUGE, CO, 2, 1>(in, aux, box, T.t[4], lb, C, k, flag, w); break;
-    default: edge_rhs_tile<GAUGE, CO, 2, 2>(in, aux, box, T.t[5], lb, C, k, flag, w); break;
+    case 0: edge_rhs_tile<GAUGE, CO, 1, 0, ODD, MIRROR>(in, aux, box, T.t[0], lb, C, k, flag, w); break;
+    case 1: edge_rhs_tile<GAUGE, CO, 1, 1, ODD, MIRROR>(in, aux, box, T.t[1], lb, C, k, flag, w); break;
+    case 2: edge_rhs_tile<GAUGE, CO, 1, 2, ODD, MIRROR>(in, aux, box, T.t[2], lb, C, k, flag, w); break;
+    case 3: edge_rhs_tile<GAUGE, CO, 2, 0, ODD, MIRROR>(in, aux, box, T.t[3], lb, C, k, flag, w); break;
+    case 4: edge_rhs_tile<GAUGE, CO, 2, 1, ODD, MIRROR>(in, aux, box, T.t[4], lb, C, k, flag, w); break;
+    default: edge_rhs_tile<GAUGE, CO, 2, 2, ODD, MIRROR>(in, aux, box, T.t[5], lb, C, k, flag, w); break;
   }
 }
 
@@ -271,10 +294,10 @@ __global__ void __launch_bounds__(kEdgeThreads) edge_update_kernel(FieldsIn u0, 
   }
 }
 
-template <int G, bool CO>
+template <int G, bool CO, bool ODD, bool MIRROR>
 void launch_edge_lds_rhs(const FieldsIn& in, const AuxOut& aux, const Box& box, const EdgeTileSet& T,
                          const Coef& C, double* K, int* flag, hipStream_t s) {
-  rhs_edge_lds_kernel<G, CO><<<(unsigned)T.tiles(), kEdgeThreads, 0, s>>>(in, aux, box, T, C, K, flag);
+  rhs_edge_lds_kernel<G, CO, ODD, MIRROR><<<(unsigned)T.tiles(), kEdgeThreads, 0, s>>>(in, aux, box, T, C, K, flag);
 }
 
 }  // namespace amss

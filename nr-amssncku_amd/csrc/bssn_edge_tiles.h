@@ -109,20 +109,54 @@ constexpr int kEdgeThreads = kEdgeTile * kEdgeTile;  // one point per thread
 AMSS_HD constexpr int edge_window_extent(int nrm, int a) {
   return a == 0 ? (nrm == 0 ? 8 : kEdgeTile + 8) : (nrm == a ? 7 : kEdgeTile + 6);
 }
-// Its layout in LDS: rows of P0 doubles (P0 >= W0: an x-normal window's
-// rows of 8 would put the neighbours along y, 16 dwords apart, on the same
-// LDS banks; rows of 10 spread them), of which the DMA fills the first W0.
-template <int NRM>
+// Its layout in LDS: rows of P0 doubles (an x-normal window's rows of 8 would
+// put the neighbours along y, 16 dwords apart, on the same LDS banks; rows of
+// 9 or 10 spread them), of which the DMA fills the first W0.  ODD: the arrays'
+// row pitch is odd, and so is P0, so that an element's LDS index and its array
+// index keep one parity along a row and between rows (the direct loads move
+// 16-byte chunks); P01 is even, and where the arrays' plane pitch is odd the
+// odd planes start one double later.
+template <int NRM, bool ODD = false>
 struct EdgeWindow {
   static constexpr int W0 = edge_window_extent(NRM, 0);
   static constexpr int W1 = edge_window_extent(NRM, 1);
   static constexpr int W2 = edge_window_extent(NRM, 2);
-  static constexpr int P0 = NRM == 0 ? W0 + 2 : W0;
-  static constexpr int P01 = P0 * W1;
-  static constexpr int NE = P01 * W2;  // doubles, row padding included
+  static constexpr int P0 = ODD ? W0 + 1 : (NRM == 0 ? W0 + 2 : W0);
+  static constexpr int P01 = ODD ? (P0 * W1 + 3) / 2 * 2 : P0 * W1;
+  static constexpr int NE = P01 * W2 + (ODD ? 2 : 0);  // doubles, padding included
   static constexpr int ROUNDS = (NE / 2 + kEdgeThreads - 1) / kEdgeThreads;  // chunks per thread
   static constexpr int PAD = 2 * ROUNDS * kEdgeThreads;                      // doubles per buffer
-  static_assert(W0 % 2 == 0 && P0 % 2 == 0, "rows of whole 16-byte chunks");
+  static_assert(W0 % 2 == 0 && P01 % 2 == 0 && P0 % 2 == (ODD ? 1 : 0), "whole 16-byte chunks");
+
+  // LDS index of window element (x, y, z): sz the arrays' plane pitch, ob 1
+  // where the window's first element is the second half of a chunk (ODD)
+  AMSS_HD static int index(int x, int y, int z, int sz, int ob) {
+    return x + y * P0 + z * P01 + (ODD ? (sz & 1 & z) + ob : 0);
+  }
+  // The array index (from the window's first element) that LDS index e, the
+  // first of a chunk, is filled from; a chunk may begin in the padding before
+  // a row (x = -1, ODD).
+  AMSS_HD static void element(int e, int sz, int ob, int& x, int& y, int& z) {
+    if (ODD) {
+      z = e / P01;
+      const int t = e - z * P01 + 1 - (sz & 1 & z) - ob;
+      y = t / P0;
+      x = t - y * P0 - 1;
+    } else {
+      x = e % P0;
+      y = (e / P0) % W1;
+      z = e / P01;
+    }
+  }
+  // Array index gi of a chunk's first element, clamped to the chunks that hold
+  // one of the array's N elements.  ODD: gi has the parity its 16-byte
+  // alignment needs; the first (last) chunk may reach one element before
+  // (past) the array, inside the same 16 bytes as its first (last) element.
+  AMSS_HD static int clamp(int gi, int N) {
+    const int lo = ODD ? -(gi & 1) : 0, hi = ODD ? N - 1 - ((gi ^ (N - 1)) & 1) : N - 2;
+    gi = gi < lo ? lo : gi;
+    return gi > hi ? hi : gi;
+  }
 };
 
 struct EdgeTiles {

@@ -101,7 +101,9 @@ struct InteriorEnv {
 // at the point's neighbour (i + di, j + dj, k + dk), which every stencil
 // here keeps within [lo, n - 1] per axis and within +-3 of the point, and
 // rel_clamped, any value of the field for a neighbour outside that range.
-template <int ORD, class D>
+// MIRROR false: the array has no symmetry plane (a point outside the interior
+// box then lacks +-3 room on some axis, and has no dissipation).
+template <int ORD, class D, bool MIRROR = true>
 struct EdgeStencils {
   static constexpr int ord = ORD;
   const Coef& C;
@@ -124,7 +126,7 @@ struct EdgeStencils {
       return i - r >= lo[0] && i + r <= n[0] - 1 && j - r >= lo[1] && j + r <= n[1] - 1 && k - r >= lo[2] &&
              k + r <= n[2] - 1;
     };
-    kook = ORD == 2 && rm(3);
+    kook = MIRROR && ORD == 2 && rm(3);
   }
   __device__ __forceinline__ const D& self() const { return *static_cast<const D*>(this); }
   __device__ double at3(int v, int di, int dj, int dk) const { return self().rel(v, di, dj, dk, 0.0); }
@@ -224,7 +226,7 @@ struct EdgeStencils {
   __device__ double ko(int v) const {
     // a point outside the interior box has +-3 room on every axis only next
     // to a symmetry plane (a uniform test before the per-point one)
-    if (lo[0] == 0 && lo[1] == 0 && lo[2] == 0) return 0.0;
+    if (!MIRROR || (lo[0] == 0 && lo[1] == 0 && lo[2] == 0)) return 0.0;
     if (!kook) return 0.0;
     const double c20 = 20.0 * at3(v, 0, 0, 0);
     double r = 0.0;

@@ -67,12 +67,11 @@ inline bool shell_on_faces(const Shell& sh, const int n[3], int mask) {
 }
 
 // Whether the LDS boundary kernels may take the order-1 and order-2 shells
-// of this box: an even row pitch (the direct loads move 16 bytes from even
-// indices), no Sommerfeld or copy face on them (a physical lower face has
+// of this box: no Sommerfeld or copy face on them (a physical lower face has
 // no mirrored halo, so its index 0 is an outermost-layer point; upper faces
 // are at n - 1), and room for their tiles in the right-hand-side buffer.
 inline bool edge_lds_ok(const Box& box, const SommerGeom& sg, const EdgeTileSet& T, const Rk4Param& R) {
-  if (!R.edge_k || (box.sy % 2) != 0 || (box.sz % 2) != 0 || T.tiles() > R.edge_k_tiles) return false;
+  if (!R.edge_k || T.tiles() > R.edge_k_tiles) return false;
   const int mask = sg.faces | sg.copy;
   for (int a = 0; a < 3; ++a)
     if (((mask >> (3 + a)) & 1) && box.mlo[a] != 0) return false;
@@ -80,11 +79,17 @@ inline bool edge_lds_ok(const Box& box, const SommerGeom& sg, const EdgeTileSet&
 }
 
 // The right-hand side on the tiles of the order-1 and order-2 shells
-// (bssn_edge_lds.h; instantiated per gauge and residual flag in
-// bssn_edge_g<G>[_res].hip), and the RK4 update of their points.
-template <int G, bool CO>
+// (bssn_edge_lds.h; instantiated in bssn_edge_inst.hip; ODD: an odd row
+// pitch; MIRROR: the array has a symmetry plane), and the RK4 update of their
+// points.
+template <int G, bool CO, bool ODD, bool MIRROR>
 void launch_edge_lds_rhs(const FieldsIn& in, const AuxOut& aux, const Box& box, const EdgeTileSet& T,
                          const Coef& C, double* K, int* flag, hipStream_t s);
+template <int G, bool CO>
+auto* edge_lds_launcher(bool odd, bool mirror) {
+  return odd ? (mirror ? launch_edge_lds_rhs<G, CO, true, true> : launch_edge_lds_rhs<G, CO, true, false>)
+             : (mirror ? launch_edge_lds_rhs<G, CO, false, true> : launch_edge_lds_rhs<G, CO, false, false>);
+}
 void launch_edge_lds_update(const FieldsIn& u0, const FieldsOut& acc, const FieldsOut& out, const AuxOut& aux,
                             const Box& box, const EdgeTileSet& T, const double* K, const Rk4Param& R,
                             hipStream_t s);
@@ -334,8 +339,9 @@ void launch_rk4_gauge(const FieldsIn& in, const FieldsIn& u0, const FieldsOut& a
       if (sh.size() <= 0 || (R.edge_order >= 0 && o != R.edge_order)) continue;
       if (lds && o >= 1) {
         if (o == 1 && ts.tiles() > 0) {
-          if (want_res) launch_edge_lds_rhs<G, true>(in, aux, box, ts, C, R.edge_k, flag, s);
-          else launch_edge_lds_rhs<G, false>(in, aux, box, ts, C, R.edge_k, flag, s);
+          const bool odd = box.sy % 2 != 0, mirror = box.mlo[0] < 0 || box.mlo[1] < 0 || box.mlo[2] < 0;
+          auto* rhs = want_res ? edge_lds_launcher<G, true>(odd, mirror) : edge_lds_launcher<G, false>(odd, mirror);
+          rhs(in, aux, box, ts, C, R.edge_k, flag, s);
           launch_edge_lds_update(u0, acc, out, aux, box, ts, R.edge_k, R, s);
         }
         continue;
