@@ -16,7 +16,7 @@ __device__ __forceinline__ bool bad_input(const FI& F, long p) {
   bool b = false;
 #pragma unroll
   for (int v = 0; v < 21; ++v) {
-    const double x = F.ptr(v)[p];
+    const double x = ((const gdouble*)F.ptr(v))[p];
     b |= !(x == x);
   }
   return b;
@@ -281,9 +281,36 @@ inline dim3 interior_grid(const Box& b) {
 inline bool box_empty(const Box& b) { return b.hi[0] <= b.lo[0] || b.hi[1] <= b.lo[1] || b.hi[2] <= b.lo[2]; }
 inline unsigned blocks_for(long n, int t) { return (unsigned)((n + t - 1) / t); }
 
+// The plain right-hand side of a whole array in one launch (bssn_rhs_lds.h;
+// instantiated in bssn_rhs_inst.hip).
+template <int G, bool CO, bool ODD>
+void launch_rhs_lds(const FieldsIn& in, const FieldsIn& mat, const FieldsOut& out, const AuxOut& aux, const Box& box,
+                    const Coef& C, int* flag, hipStream_t s);
+
+// Whether it may run: no symmetry plane (the variant with the mirror pass,
+// whose point computations spilled most, gave wrong values and was not kept),
+// every axis of 5 points or more (the boundary tiles' windows are laid out
+// for those), 32-bit byte offsets, and with an even row
+// pitch every state array on 16 bytes (the direct loads' alignment; with an
+// odd pitch the layout follows each array's own).
+inline bool rhs_lds_ok(const FieldsIn& in, const Box& box) {
+  for (int a = 0; a < 3; ++a)
+    if (box.n[a] < 5 || box.mlo[a] < 0) return false;
+  if ((long)box.n[0] * box.n[1] * box.n[2] >= (1L << 29)) return false;
+  for (int v = 0; v < NFIELD; ++v)
+    if (((uintptr_t)in.p[v]) % (box.sy % 2 == 0 ? 16 : 8) != 0) return false;
+  return true;
+}
+
 template <int G>
 void launch_rhs_gauge(const FieldsIn& in, const FieldsIn& mat, const FieldsOut& out, const AuxOut& aux,
                       const Box& box, const Coef& C, int co, int* flag, bool edge, hipStream_t s) {
+  if (edge && rhs_lds_ok(in, box)) {
+    auto* rhs = box.sy % 2 != 0 ? (co == 0 ? launch_rhs_lds<G, true, true> : launch_rhs_lds<G, false, true>)
+                                : (co == 0 ? launch_rhs_lds<G, true, false> : launch_rhs_lds<G, false, false>);
+    rhs(in, mat, out, aux, box, C, flag, s);
+    return;
+  }
   if (co == 0) {
     if (!box_empty(box)) rhs_interior_kernel<G, true><<<interior_grid(box), kRhsThreads, 0, s>>>(in, mat, out, aux, box, C, flag);
   } else {
