@@ -62,172 +62,239 @@ int xfer_plan(const double* llbc, const double* uubc, const int* extc, const dou
   return 0;
 }
 
-// The source value at 1-based index q (symmetry_bd's mirror below 1:
-// q -> 1 - q with the parity of each mirrored axis, fmisc.f90:877-901).
-struct XferSrc {
-  const double* __restrict__ f;
-  int n0, n1;
-  double S[3];
-  __device__ __forceinline__ double at(int i, int j, int k) const {
-    double s = 1.0;
-    if (i < 1) { i = 1 - i; s *= S[0]; }
-    if (j < 1) { j = 1 - j; s *= S[1]; }
-    if (k < 1) { k = 1 - k; s *= S[2]; }
-    return f[(i - 1) + (long)n0 * ((j - 1) + (long)n1 * (k - 1))] * s;
-  }
-};
-
-// Both transfers work on tiles of target cells: the source block a tile
-// needs is staged once in LDS and the 6x6x6 contraction is factorized (along
-// z for every (y, x) of the block, then along y, then along x), which is
-// the reference's summation order.  Cells past the end of the target range
-// in a partial tile are computed from unloaded LDS and not stored; every LDS
-// index stays inside the fixed block sizes (shown at each size below).
+// Both transfers work on tiles of target cells and factorize the 6x6x6
+// contraction along z, then y, then x (the reference's summation order).  A
+// thread takes a whole column of the source block in z -- all its loads in
+// flight together, coalesced along x -- and forms the tile's values along z
+// from registers; y and x follow through LDS the same way.  Bound by the
+// latency of one such round trip per tile (an 8-16 deep chain of loads, two
+// barriers) and by the launch, not by bytes: the earlier kernels staged the
+// block in LDS in a loop whose every load waited.  A 134^3 fine array takes
+// 12.9 us (36 before; its 9 bytes a cell 3.8 us at the rate of a copy), 62^3
+// coarse cells 11.4 us (28).
+// blockIdx.y is the field, blockIdx.x a tile of one of the regions.
+// Source cells past what the valid target cells read are clamped or skipped;
+// cells past the end of the target range are not stored.
 constexpr double kProW[6] = {77.0 / 8192.0, -693.0 / 8192.0, 3465.0 / 4096.0,
                              1155.0 / 4096.0, -495.0 / 8192.0, 63.0 / 8192.0};
 constexpr double kResW[3] = {3.0 / 256.0, -25.0 / 256.0, 75.0 / 128.0};
 
-// prolong: fine tile 16 x 8 x 8.  Fine cell p reads coarse cells
-// c(p) - 2 .. c(p) + 3, c(p) = (p + lbf - 1) / 2 - lbc + 1; over a tile c
-// advances by at most (F - 1 + 1) / 2 = F / 2, so a block of F / 2 + 6 coarse
-// cells per axis covers it (index c(p) - c(p0) + q <= F / 2 + 5).
-constexpr int kPFX = 16, kPFY = 8, kPFZ = 8;
-constexpr int kPCX = kPFX / 2 + 6, kPCY = kPFY / 2 + 6, kPCZ = kPFZ / 2 + 6;
+namespace {
 
-__global__ void __launch_bounds__(256) prolong3_kernel(XferSrc src, double* __restrict__ funf, XferPlan P) {
-  __shared__ double B[kPCZ][kPCY][kPCX];
+// A column of the source at 1-based (i, j), cells k0, k0 + 1, ... (at most
+// kmax): symmetry_bd's mirror below 1 (q -> 1 - q with the parity of each
+// mirrored axis, fmisc.f90:877-901).
+template <int N>
+__device__ __forceinline__ void load_column(const XferField& F, int n0, int n1, int i, int j, int k0, int kmax,
+                                            double (&c)[N]) {
+  double s = 1.0;
+  if (i < 1) { i = 1 - i; s *= F.S[0]; }
+  if (j < 1) { j = 1 - j; s *= F.S[1]; }
+  const double* f = F.src + (i - 1) + (long)n0 * (j - 1);
+  const long nz = (long)n0 * n1;
+#pragma unroll
+  for (int q = 0; q < N; ++q) {
+    const int k = min(k0 + q, kmax);
+    const double v = f[nz * (k < 1 ? -k : k - 1)];
+    c[q] = v * (k < 1 ? s * F.S[2] : s);
+  }
+}
+
+// Fine values d = 0 .. 7 of a line whose first fine cell has an even (odd)
+// global index, from coarse values c: cell d reads c[o .. o + 5], o = (ODD + d)
+// / 2, with the weights in reverse order on odd cells.
+template <bool ODD, int N>
+__device__ __forceinline__ void prolong_line(const double (&c)[10], double (&f)[N]) {
+#pragma unroll
+  for (int d = 0; d < N; ++d) {
+    const int g = ODD + d, o = g / 2;
+    double s = 0.0;
+#pragma unroll
+    for (int q = 0; q < 6; ++q) s += kProW[(g & 1) ? 5 - q : q] * c[o + q];
+    f[d] = s;
+  }
+}
+template <int N>
+__device__ __forceinline__ void prolong_line(bool odd, const double (&c)[10], double (&f)[N]) {
+  if (odd) prolong_line<true, N>(c, f);
+  else prolong_line<false, N>(c, f);
+}
+
+// the region of block b, and b's tile in it
+__device__ __forceinline__ const XferPlan& xfer_region(const XferBatch& X, int& b) {
+  int r = 0;
+  while (r + 1 < X.nregion && b >= X.first[r + 1]) ++r;
+  b -= X.first[r];
+  return X.P[r];
+}
+
+}  // namespace
+
+// prolong: fine tile 32 x 8 x 8.  Fine cell p reads coarse cells
+// c(p) - 2 .. c(p) + 3, c(p) = (p + lbf - 1) / 2 - lbc + 1; over a tile of F
+// cells c advances by at most F / 2, so F / 2 + 6 coarse cells cover it.
+constexpr int kPFX = 32, kPFY = 8, kPFZ = 8;
+constexpr int kPCX = kPFX / 2 + 6, kPCY = kPFY / 2 + 6;
+static_assert(kPFY / 2 + 6 == 10 && kPFZ / 2 + 6 == 10, "prolong_line reads 10 coarse values");
+
+__global__ void __launch_bounds__(256) prolong3_kernel(XferBatch X) {
   __shared__ double T1[kPFZ][kPCY][kPCX];
   __shared__ double T2[kPFZ][kPFY][kPCX];
-  const int F[3] = {kPFX, kPFY, kPFZ};
-  int nt[3], p0[3], pe[3], c0[3], par0[3];
-  for (int a = 0; a < 3; ++a) nt[a] = (P.hi[a] - P.lo[a] + F[a]) / F[a];
-  const int b = blockIdx.x;
+  int b = blockIdx.x;
+  const XferPlan& P = xfer_region(X, b);
+  const XferField& F = X.f[blockIdx.y];
+  const int T[3] = {kPFX, kPFY, kPFZ};
+  int nt[3], p0[3], pe[3], c0[3], nc[3];
+  bool odd[3];  // parity of the tile's first fine cell
+  for (int a = 0; a < 3; ++a) nt[a] = (P.hi[a] - P.lo[a] + T[a]) / T[a];
   const int tb[3] = {b % nt[0], (b / nt[0]) % nt[1], b / (nt[0] * nt[1])};
   for (int a = 0; a < 3; ++a) {
-    p0[a] = P.lo[a] + tb[a] * F[a];
-    pe[a] = min(p0[a] + F[a] - 1, P.hi[a]);
-    c0[a] = (p0[a] + P.lbf[a] - 1) / 2 - P.lbc[a] + 1;
-    par0[a] = p0[a] + P.lbf[a] - 1;  // fine global index of p0 (its parity picks the weights)
+    p0[a] = P.lo[a] + tb[a] * T[a];
+    pe[a] = min(p0[a] + T[a] - 1, P.hi[a]);
+    const int g = p0[a] + P.lbf[a] - 1;
+    odd[a] = g & 1;
+    c0[a] = g / 2 - P.lbc[a] + 1 - 2;  // first coarse cell of the block
+    nc[a] = (pe[a] + P.lbf[a] - 1) / 2 - P.lbc[a] + 1 + 3 - c0[a] + 1;  // ... that the valid fine cells read
   }
   const int tid = threadIdx.x;
-  // the coarse cells the tile's valid fine cells read, mirrored below 1
-  int nc[3];
-  for (int a = 0; a < 3; ++a) nc[a] = ((pe[a] + P.lbf[a] - 1) / 2 - P.lbc[a] + 1) + 3 - (c0[a] - 2) + 1;
-  for (int e = tid; e < nc[0] * nc[1] * nc[2]; e += 256) {
-    const int x = e % nc[0], y = (e / nc[0]) % nc[1], z = e / (nc[0] * nc[1]);
-    B[z][y][x] = src.at(c0[0] - 2 + x, c0[1] - 2 + y, c0[2] - 2 + z);
+  if (tid < kPCX * kPCY) {
+    const int x = tid % kPCX, y = tid / kPCX;
+    if (x < nc[0] && y < nc[1]) {
+      double c[10], f[kPFZ];
+      load_column(F, P.ext_c[0], P.ext_c[1], c0[0] + x, c0[1] + y, c0[2], c0[2] + nc[2] - 1, c);
+      prolong_line(odd[2], c, f);
+#pragma unroll
+      for (int d = 0; d < kPFZ; ++d) T1[d][y][x] = f[d];
+    }
   }
   __syncthreads();
-  // offset of fine cell d of the tile in the block, and its weight order
-  auto off = [&](int a, int d) { return (par0[a] + d) / 2 - par0[a] / 2; };
-  auto rev = [&](int a, int d) { return ((par0[a] + d) & 1) != 0; };
-  for (int e = tid; e < kPFZ * kPCY * kPCX; e += 256) {
-    const int x = e % kPCX, y = (e / kPCX) % kPCY, fz = e / (kPCX * kPCY);
-    const int o = off(2, fz);
-    const bool r = rev(2, fz);
-    double s = 0.0;
-    for (int q = 0; q < 6; ++q) s += kProW[r ? 5 - q : q] * B[o + q][y][x];
-    T1[fz][y][x] = s;
+  if (tid < kPCX * kPFZ) {
+    const int x = tid % kPCX, z = tid / kPCX;
+    double c[10], f[kPFY];
+#pragma unroll
+    for (int q = 0; q < 10; ++q) c[q] = T1[z][q][x];
+    prolong_line(odd[1], c, f);
+#pragma unroll
+    for (int d = 0; d < kPFY; ++d) T2[z][d][x] = f[d];
   }
   __syncthreads();
-  for (int e = tid; e < kPFZ * kPFY * kPCX; e += 256) {
-    const int x = e % kPCX, fy = (e / kPCX) % kPFY, fz = e / (kPCX * kPFY);
-    const int o = off(1, fy);
-    const bool r = rev(1, fy);
+  const int fx = tid % kPFX, fy = tid / kPFX, g = (odd[0] ? 1 : 0) + fx, o = g / 2;
+  const int i = p0[0] + fx, j = p0[1] + fy;
+  if (i > pe[0] || j > pe[1]) return;
+  double w[6];
+#pragma unroll
+  for (int q = 0; q < 6; ++q) w[q] = (g & 1) ? kProW[5 - q] : kProW[q];
+  double* out = F.dst + (i - 1) + (long)P.ext_f[0] * (j - 1);
+  const long nz = (long)P.ext_f[0] * P.ext_f[1];
+#pragma unroll
+  for (int fz = 0; fz < kPFZ; ++fz) {
     double s = 0.0;
-    for (int q = 0; q < 6; ++q) s += kProW[r ? 5 - q : q] * T1[fz][o + q][x];
-    T2[fz][fy][x] = s;
-  }
-  __syncthreads();
-  for (int e = tid; e < kPFZ * kPFY * kPFX; e += 256) {
-    const int fx = e % kPFX, fy = (e / kPFX) % kPFY, fz = e / (kPFX * kPFY);
-    const int o = off(0, fx);
-    const bool r = rev(0, fx);
-    double s = 0.0;
-    for (int q = 0; q < 6; ++q) s += kProW[r ? 5 - q : q] * T2[fz][fy][o + q];
-    const int i = p0[0] + fx, j = p0[1] + fy, k = p0[2] + fz;
-    if (i <= pe[0] && j <= pe[1] && k <= pe[2])
-      funf[(i - 1) + (long)P.ext_f[0] * ((j - 1) + (long)P.ext_f[1] * (k - 1))] = s;
+#pragma unroll
+    for (int q = 0; q < 6; ++q) s += w[q] * T2[fz][fy][o + q];
+    if (p0[2] + fz <= pe[2]) out[nz * (p0[2] + fz - 1)] = s;
   }
 }
 
-// restrict: coarse tile 8 x 8 x 4.  Coarse cell p reads fine cells
+// restrict: coarse tile 16 x 4 x 4.  Coarse cell p reads fine cells
 // f(p) - 2 .. f(p) + 3, f(p) = 2 (p + lbc - 1) - lbf; over a tile f advances
-// by 2 per cell, so a block of 2 C + 4 fine cells per axis covers it
-// (index 2 d + q <= 2 C + 3).
-constexpr int kRCX = 8, kRCY = 8, kRCZ = 4;
+// by 2 per cell, so a block of 2 C + 4 fine cells per axis covers it.
+constexpr int kRCX = 16, kRCY = 4, kRCZ = 4;
 constexpr int kRFX = 2 * kRCX + 4, kRFY = 2 * kRCY + 4, kRFZ = 2 * kRCZ + 4;
 
-__global__ void __launch_bounds__(256) restrict3_kernel(XferSrc src, double* __restrict__ func, XferPlan P) {
-  __shared__ double B[kRFZ][kRFY][kRFX];
+template <int N>
+__device__ __forceinline__ void restrict_line(const double (&f)[2 * N + 4], double (&c)[N]) {
+#pragma unroll
+  for (int d = 0; d < N; ++d)
+    c[d] = kResW[0] * (f[2 * d] + f[2 * d + 5]) + kResW[1] * (f[2 * d + 1] + f[2 * d + 4]) +
+           kResW[2] * (f[2 * d + 2] + f[2 * d + 3]);
+}
+
+__global__ void __launch_bounds__(256) restrict3_kernel(XferBatch X) {
   __shared__ double T1[kRCZ][kRFY][kRFX];
   __shared__ double T2[kRCZ][kRCY][kRFX];
-  const int Ct[3] = {kRCX, kRCY, kRCZ};
-  int nt[3], p0[3], pe[3], f0[3];
-  for (int a = 0; a < 3; ++a) nt[a] = (P.hi[a] - P.lo[a] + Ct[a]) / Ct[a];
-  const int b = blockIdx.x;
+  int b = blockIdx.x;
+  const XferPlan& P = xfer_region(X, b);
+  const XferField& F = X.f[blockIdx.y];
+  const int T[3] = {kRCX, kRCY, kRCZ};
+  int nt[3], p0[3], pe[3], f0[3], nf[3];
+  for (int a = 0; a < 3; ++a) nt[a] = (P.hi[a] - P.lo[a] + T[a]) / T[a];
   const int tb[3] = {b % nt[0], (b / nt[0]) % nt[1], b / (nt[0] * nt[1])};
   for (int a = 0; a < 3; ++a) {
-    p0[a] = P.lo[a] + tb[a] * Ct[a];
-    pe[a] = min(p0[a] + Ct[a] - 1, P.hi[a]);
-    f0[a] = 2 * (p0[a] + P.lbc[a] - 1) - P.lbf[a];
+    p0[a] = P.lo[a] + tb[a] * T[a];
+    pe[a] = min(p0[a] + T[a] - 1, P.hi[a]);
+    f0[a] = 2 * (p0[a] + P.lbc[a] - 1) - P.lbf[a] - 2;  // first fine cell of the block
+    nf[a] = 2 * (pe[a] - p0[a]) + 6;                    // ... that the valid coarse cells read
   }
   const int tid = threadIdx.x;
-  int nf[3];
-  for (int a = 0; a < 3; ++a) nf[a] = 2 * (pe[a] - p0[a]) + 6;
-  for (int e = tid; e < nf[0] * nf[1] * nf[2]; e += 256) {
-    const int x = e % nf[0], y = (e / nf[0]) % nf[1], z = e / (nf[0] * nf[1]);
-    B[z][y][x] = src.at(f0[0] - 2 + x, f0[1] - 2 + y, f0[2] - 2 + z);
+#pragma unroll
+  for (int e = 0; e < kRFX * kRFY; e += 256) {
+    const int x = (e + tid) % kRFX, y = (e + tid) / kRFX;
+    if (x < nf[0] && y < nf[1]) {
+      double f[kRFZ], c[kRCZ];
+      load_column(F, P.ext_f[0], P.ext_f[1], f0[0] + x, f0[1] + y, f0[2], f0[2] + nf[2] - 1, f);
+      restrict_line(f, c);
+#pragma unroll
+      for (int d = 0; d < kRCZ; ++d) T1[d][y][x] = c[d];
+    }
   }
   __syncthreads();
-  for (int e = tid; e < kRCZ * kRFY * kRFX; e += 256) {
-    const int x = e % kRFX, y = (e / kRFX) % kRFY, cz = e / (kRFX * kRFY);
-    const double* v = &B[2 * cz][y][x];
-    constexpr int S = kRFY * kRFX;
-    T1[cz][y][x] = kResW[0] * (v[0] + v[5 * S]) + kResW[1] * (v[S] + v[4 * S]) + kResW[2] * (v[2 * S] + v[3 * S]);
+  if (tid < kRFX * kRCZ) {
+    const int x = tid % kRFX, z = tid / kRFX;
+    double f[kRFY], c[kRCY];
+#pragma unroll
+    for (int q = 0; q < kRFY; ++q) f[q] = T1[z][q][x];
+    restrict_line(f, c);
+#pragma unroll
+    for (int d = 0; d < kRCY; ++d) T2[z][d][x] = c[d];
   }
   __syncthreads();
-  for (int e = tid; e < kRCZ * kRCY * kRFX; e += 256) {
-    const int x = e % kRFX, cy = (e / kRFX) % kRCY, cz = e / (kRFX * kRCY);
-    const double* v = &T1[cz][2 * cy][x];
-    constexpr int S = kRFX;
-    T2[cz][cy][x] = kResW[0] * (v[0] + v[5 * S]) + kResW[1] * (v[S] + v[4 * S]) + kResW[2] * (v[2 * S] + v[3 * S]);
-  }
-  __syncthreads();
-  {
-    const int cx = tid % kRCX, cy = (tid / kRCX) % kRCY, cz = tid / (kRCX * kRCY);
-    const double* v = &T2[cz][cy][2 * cx];
-    const double r = kResW[0] * (v[0] + v[5]) + kResW[1] * (v[1] + v[4]) + kResW[2] * (v[2] + v[3]);
-    const int i = p0[0] + cx, j = p0[1] + cy, k = p0[2] + cz;
-    if (i <= pe[0] && j <= pe[1] && k <= pe[2])
-      func[(i - 1) + (long)P.ext_c[0] * ((j - 1) + (long)P.ext_c[1] * (k - 1))] = r;
-  }
+  const int cx = tid % kRCX, cy = (tid / kRCX) % kRCY, cz = tid / (kRCX * kRCY);
+  const double* v = &T2[cz][cy][2 * cx];
+  const double r = kResW[0] * (v[0] + v[5]) + kResW[1] * (v[1] + v[4]) + kResW[2] * (v[2] + v[3]);
+  const int i = p0[0] + cx, j = p0[1] + cy, k = p0[2] + cz;
+  if (i <= pe[0] && j <= pe[1] && k <= pe[2])
+    F.dst[(i - 1) + (long)P.ext_c[0] * ((j - 1) + (long)P.ext_c[1] * (k - 1))] = r;
 }
 
-// target points of a plan; 0 when any axis is empty (nothing is launched)
-static long plan_points(const XferPlan& P) {
-  long n = 1;
-  for (int a = 0; a < 3; ++a) n *= P.hi[a] >= P.lo[a] ? (long)(P.hi[a] - P.lo[a] + 1) : 0L;
-  return n;
+static_assert(kRCX * kRCY * kRCZ == 256 && kPFX * kPFY == 256, "one target column or cell per thread");
+
+// The tiles (of size T) of a batch's regions; empty regions give none.
+static unsigned batch_tiles(XferBatch& X, const int T[3]) {
+  int first = 0;
+  for (int r = 0; r < X.nregion; ++r) {
+    const XferPlan& P = X.P[r];
+    int n = 1;
+    for (int a = 0; a < 3; ++a) n *= P.hi[a] >= P.lo[a] ? (P.hi[a] - P.lo[a] + T[a]) / T[a] : 0;
+    X.first[r] = first;
+    first += n;
+  }
+  return (unsigned)first;
 }
 
-// tiles of size T covering the target range of a plan
-static unsigned plan_tiles(const XferPlan& P, const int T[3]) {
-  long n = 1;
-  for (int a = 0; a < 3; ++a) n *= (P.hi[a] - P.lo[a] + T[a]) / T[a];
-  return (unsigned)n;
+void launch_prolong3(XferBatch X, hipStream_t s) {
+  const int T[3] = {kPFX, kPFY, kPFZ};
+  const unsigned n = batch_tiles(X, T);
+  if (n > 0 && X.nfield > 0) prolong3_kernel<<<dim3(n, X.nfield), 256, 0, s>>>(X);
+}
+
+void launch_restrict3(XferBatch X, hipStream_t s) {
+  const int T[3] = {kRCX, kRCY, kRCZ};
+  const unsigned n = batch_tiles(X, T);
+  if (n > 0 && X.nfield > 0) restrict3_kernel<<<dim3(n, X.nfield), 256, 0, s>>>(X);
 }
 
 void launch_prolong3(const double* func, double* funf, const XferPlan& P, const double S[3], hipStream_t s) {
-  const int T[3] = {kPFX, kPFY, kPFZ};
-  XferSrc src{func, P.ext_c[0], P.ext_c[1], {S[0], S[1], S[2]}};
-  if (plan_points(P) > 0) prolong3_kernel<<<plan_tiles(P, T), 256, 0, s>>>(src, funf, P);
+  XferBatch X;
+  X.add(P);
+  X.add(func, funf, S);
+  launch_prolong3(X, s);
 }
 
 void launch_restrict3(const double* funf, double* func, const XferPlan& P, const double S[3], hipStream_t s) {
-  const int T[3] = {kRCX, kRCY, kRCZ};
-  XferSrc src{funf, P.ext_f[0], P.ext_f[1], {S[0], S[1], S[2]}};
-  if (plan_points(P) > 0) restrict3_kernel<<<plan_tiles(P, T), 256, 0, s>>>(src, func, P);
+  XferBatch X;
+  X.add(P);
+  X.add(funf, func, S);
+  launch_restrict3(X, s);
 }
 
 }  // namespace amss
