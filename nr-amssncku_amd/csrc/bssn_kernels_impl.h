@@ -140,28 +140,46 @@ AMSS_POINT_KERNEL rk4_interior_kernel(FieldsIn in, FieldsIn u0, FieldsOut acc, F
   S.finish();
 }
 
-// LDS-staged variant: 8x8xTZ-point tiles, halo tiles of every field group in
-// LDS (double-buffered, filled by direct global->LDS loads).  A 1-D grid of
-// tiles in XCD-contiguous order: consecutive tiles, whose halos overlap, run
-// behind the same L2.  The tiles cover the box whole: threads of a partial
-// tile past it compute on a clamped point and store nothing (remainder slabs
-// on the direct kernel took 120-155 us each and sub-step, whatever their size:
-// a coarse step of a 64^3 patch and a nested one of 76^3 with them 10.2 ms,
-// with partial tiles 7.4 ms).  The 8-deep tile
-// (512 threads, one workgroup per CU) re-reads 14/8 instead of 10/4 z-planes
-// of halo per interior plane.  Instantiated in bssn_lds_g<G>[_odd].hip.
+// LDS-staged variant: tiles of a shape in kLdsShape, halo tiles of every
+// field group in LDS (double-buffered, filled by direct global->LDS loads).  A
+// 1-D grid of tiles in XCD-contiguous order: consecutive tiles, whose halos
+// overlap, run behind the same L2.  The tiles cover the box whole: threads of
+// a partial tile past it compute on a clamped point and store nothing
+// (remainder slabs on the direct kernel took 120-155 us each and sub-step,
+// whatever their size: a coarse step of a 64^3 patch and a nested one of 76^3
+// with them 10.2 ms, with partial tiles 7.4 ms).  Instantiated in
+// bssn_lds_g<G>[_odd].hip; lds_tile_shape (bssn_lds_launch.h) picks the shape.
 constexpr int kLdsTX = 8, kLdsTY = 8, kLdsTZ = 4;
+constexpr int kLdsShape[3][3] = {{8, 8, 4}, {8, 8, 8}, {32, 4, 4}};
+// Tile b of gx x gy x gz: x fastest, then y in strips of `strip` tiles, then
+// z, then the strips, so that the tiles an XCD holds at a time (32 of 512
+// points) form a block whose halo is small: 128 x 16 x 8 points of 4 x 4 x 2
+// wide tiles, 16 x 2 of cubic ones, at 128 points per row.  Sub-step 1 of 128^3
+// points in 32x4x4 tiles: 993 us in plain order, 975 / 951 / 972 in strips of
+// 2 / 4 / 8.  What bounds the kernel there is memory traffic: 4.3-4.6 GB per
+// launch in 0.89-0.92 ms, 4.8 TB/s where a copy reaches 5.7.  The halo is read
+// 5.7 times over the state's own bytes, as an XCD's tiles drift apart and its L2
+// forgets; holding each 32 tiles together by a counter took 12% off the reads
+// and cost 7% of the time, all of them then loading at once.
+__device__ __forceinline__ void tile_place(int b, int gx, int gy, int gz, int strip, int& x, int& y, int& z) {
+  const int full = gx * strip * gz, s = b / full, r = b - s * full, h = min(strip, gy - s * strip);
+  x = r % gx;
+  y = s * strip + (r / gx) % h;
+  z = r / (gx * h);
+}
 #ifndef AMSS_LDS_WAVES
 #define AMSS_LDS_WAVES 2
 #endif
-template <int GAUGE, int STAGE, bool CO, int TZ, bool ODD>
-__global__ void __launch_bounds__(kLdsTX * kLdsTY * TZ) __attribute__((amdgpu_waves_per_eu(AMSS_LDS_WAVES, AMSS_LDS_WAVES)))
+template <int GAUGE, int STAGE, bool CO, int SH, bool ODD>
+__global__ void __launch_bounds__(kLdsShape[SH][0] * kLdsShape[SH][1] * kLdsShape[SH][2])
+    __attribute__((amdgpu_waves_per_eu(AMSS_LDS_WAVES, AMSS_LDS_WAVES)))
 rk4_lds_kernel(FieldsIn in, FieldsIn u0, FieldsOut acc, FieldsOut out, AuxOut aux, Box box,
                                  Coef C, Rk4Param R, int* flag, long nfill) {
-  using Tl = LdsTile<kLdsTX, kLdsTY, TZ, ODD>;
+  constexpr int TX = kLdsShape[SH][0], TY = kLdsShape[SH][1], TZ = kLdsShape[SH][2];
+  using Tl = LdsTile<TX, TY, TZ, ODD>;
   __shared__ __attribute__((aligned(16))) double tiles[kLdsBuffers * Tl::NPAD];
-  const int gx = (box.hi[0] - box.lo[0] + kLdsTX - 1) / kLdsTX, gy = (box.hi[1] - box.lo[1] + kLdsTY - 1) / kLdsTY;
-  const int ntiles = gx * gy * ((box.hi[2] - box.lo[2] + TZ - 1) / TZ);
+  const int gx = (box.hi[0] - box.lo[0] + TX - 1) / TX, gy = (box.hi[1] - box.lo[1] + TY - 1) / TY;
+  const int gz = (box.hi[2] - box.lo[2] + TZ - 1) / TZ, ntiles = gx * gy * gz;
   if ((int)blockIdx.x >= ntiles) {
     // the frozen-ghost fill of the nfill points outside [3, n - 3) of the
     // array (nfill is 0 when the caller fills them), in the workgroups after
@@ -179,14 +197,14 @@ rk4_lds_kernel(FieldsIn in, FieldsIn u0, FieldsOut acc, FieldsOut out, AuxOut au
   }
   int tx, ty, tz;
   Tl::point((int)threadIdx.x, tx, ty, tz);
-  const int b = xcd_spread(blockIdx.x, ntiles);
-  const int i0 = box.lo[0] + (b % gx) * kLdsTX, j0 = box.lo[1] + ((b / gx) % gy) * kLdsTY;
-  const int k0 = box.lo[2] + (b / (gx * gy)) * TZ;
+  int bx, by, bz;
+  tile_place(xcd_spread(blockIdx.x, ntiles), gx, gy, gz, TX == 32 ? 4 : gy, bx, by, bz);
+  const int i0 = box.lo[0] + bx * TX, j0 = box.lo[1] + by * TY, k0 = box.lo[2] + bz * TZ;
   const int N = box.n[0] * box.n[1] * box.n[2];
   bool live;
   const BufIo io = tile_io(i0 + tx, j0 + ty, k0 + tz, box.hi[0], box.hi[1], box.hi[2], (int)box.sy, (int)box.sz, N, live);
   lds_double* t0 = (lds_double*)tiles;
-  LdsRk4<STAGE, kLdsTX, kLdsTY, TZ, FieldsIn, FieldsOut, AuxOut, true, ODD> X{
+  LdsRk4<STAGE, TX, TY, TZ, FieldsIn, FieldsOut, AuxOut, true, ODD> X{
       {in, in, C, t0, t0 + (kLdsBuffers / 2) * Tl::NPAD, io, Tl::lds_index(tx, ty, tz, (int)box.sz),
        (int)((i0 - 3) + (j0 - 3) * box.sy + (k0 - 3) * box.sz), (int)box.sy, (int)box.sz, N, (int)threadIdx.x, tz + 3},
       {u0, acc, out, aux, io, R.c, R.tinny, {}}};

@@ -50,36 +50,40 @@ __host__ __device__ constexpr int tile_row(int r, int TY) { return TY == 8 ? ((r
 // parity throughout the tile.
 //  EVEN row pitch of the arrays: rows of TX + 6 doubles, planes without gaps
 //    (rows start at an even x, and so does every chunk).
-//  ODD pitch: rows of 15 doubles (elements x = -1 .. 13; -1 is padding whose
-//    chunk may hold it and x = 0), planes of 216 (16 banks apart, so that a
-//    wave of 8 x 4 x 2 points has each 16-lane access group -- 8 points of x
-//    on two planes -- on disjoint banks); where the arrays' plane pitch is odd
-//    too, odd planes start one double later.  A sub-step of 85^3 points takes
-//    395 us (the direct kernel, which took odd pitches before, about 650); the
-//    same tiles filled by 4-byte loads spilled scalar registers (730 us with
-//    the residuals).
+//  ODD pitch: rows one double longer (elements x = -1 .. TX + 5; -1 is padding
+//    whose chunk may hold it and x = 0), planes of an even pitch with room for
+//    one more; where the arrays' plane pitch is odd too, odd planes start one
+//    double later.  A sub-step of 85^3 points takes 395 us on 8x8x8 tiles (the
+//    direct kernel, which took odd pitches before, about 650); the same tiles
+//    filled by 4-byte loads spilled scalar registers (730 us with the
+//    residuals).
+// LDS banks: a ds_read_b64 serves 16 lanes at a time.  Rows of 16 points or
+// more need no care; an 8-point row pairs with one 16 banks away: row y + 4
+// (EVEN, tile_row), or the same row of plane z + 1 (ODD: planes of 216
+// doubles, a wave of 8 x 4 x 2 points).
 template <int TX, int TY, int TZ, bool ODD = false>
 struct LdsTile {
   static constexpr int LX = TX + 6, LY = TY + 6, LZ = TZ + 6;
-  static constexpr int PY = ODD ? LX + 1 : LX, PZ = ODD ? 216 : LX * LY;  // LDS pitches
+  static constexpr int PY = ODD ? LX + 1 : LX;  // LDS pitches
+  static constexpr int PZ = !ODD ? LX * LY : (TX == 8 ? 216 : (PY * LY + 3) / 2 * 2);
   static constexpr int NCH = PZ * LZ / 2;  // 16-byte chunks
   static constexpr int NT = TX * TY * TZ;  // threads
   static constexpr int ROUNDS = (NCH + NT - 1) / NT;
   static constexpr int NPAD = 2 * ROUNDS * NT;  // doubles per buffer: whole rounds, no bounds branches
   static_assert(LX % 2 == 0, "tile rows must hold whole 16-byte chunks");
   static_assert(NT % 64 == 0, "whole waves");
-  static_assert(!ODD || (TX == 8 && TY == 8 && PY * LY + 2 <= PZ), "odd pitch: 8 x 8 rows");
-  static_assert(PZ * LZ < NPAD || !ODD, "room for the last plane's shift");
+  static_assert(!ODD || (PZ % 2 == 0 && PY * LY + 2 <= PZ && PZ * LZ < NPAD), "room for the shifts");
+  static_assert(!ODD || TX >= 16 || (TX == 8 && TY == 8), "odd pitch: 8 x 8 rows or wide ones");
 
   // the tile point of thread tid
   __device__ __forceinline__ static void point(int tid, int& tx, int& ty, int& tz) {
-    if (ODD) {
+    if (ODD && TX == 8) {
       tx = tid & 7;
       ty = ((tid >> 4) & 3) + 4 * ((tid >> 6) & 1);
       tz = ((tid >> 3) & 1) + 2 * (tid >> 7);
     } else {
       tx = tid % TX;
-      ty = tile_row((tid / TX) % TY, TY);
+      ty = TX <= 8 ? tile_row((tid / TX) % TY, TY) : (tid / TX) % TY;
       tz = tid / (TX * TY);
     }
   }
@@ -111,9 +115,17 @@ constexpr int kLdsBuffers = AMSS_LDS_PAIRS ? 4 : 2;
 #ifndef AMSS_TOP
 #define AMSS_TOP 1
 #endif
-#ifndef AMSS_DMA_AT
-#define AMSS_DMA_AT 1
-#endif
+// When a pair's two halo tiles are issued, one pair ahead: both at the barrier
+// (0), the first there and the second with the second group (1), both with the
+// second group (2).  Self::kDmaAt says; 1 by default.
+template <class S, class = void>
+struct DmaAt {
+  static constexpr int v = 1;
+};
+template <class S>
+struct DmaAt<S, std::void_t<decltype(S::kDmaAt)>> {
+  static constexpr int v = S::kDmaAt;
+};
 // Self: a type deriving from this environment and from the RK4 epilogue,
 // whose prefetch(v0, v1) the environment calls for each pair (void: none).
 template <int TX, int TY, int TZ, class FI = FieldsIn, class Self = void, bool ODD = false>
@@ -222,6 +234,7 @@ struct LdsEnv {
     if (AMSS_LDS_PAIRS) issue(group_field(1), slot(1));
   }
   __device__ __forceinline__ void begin(int v) {
+    constexpr int kAt = DmaAt<Self>::v;
     if (!AMSS_LDS_PAIRS) {
       __builtin_amdgcn_s_waitcnt(0);
       __syncthreads();
@@ -233,13 +246,13 @@ struct LdsEnv {
       if (g + 2 < NFIELD) ahead(g + 2);
       __builtin_amdgcn_sched_barrier(0);
       if (g + 2 < NFIELD) {
-        if (AMSS_DMA_AT < 2) issue(group_field(g + 2), slot(g + 2));
-        if (AMSS_DMA_AT < 1) issue(group_field(g + 3), slot(g + 3));
+        if (kAt < 2) issue(group_field(g + 2), slot(g + 2));
+        if (kAt < 1) issue(group_field(g + 3), slot(g + 3));
       }
-    } else if (AMSS_DMA_AT > 0 && g + 1 < NFIELD) {
+    } else if (kAt > 0 && g + 1 < NFIELD) {
       // the next pair's halo loads start with the pair's second group
       __builtin_amdgcn_sched_barrier(0);
-      if (AMSS_DMA_AT > 1) issue(group_field(g + 1), slot(g + 1));
+      if (kAt > 1) issue(group_field(g + 1), slot(g + 1));
       issue(group_field(g + 2), slot(g + 2));
       __builtin_amdgcn_sched_barrier(0);
     }
@@ -343,6 +356,10 @@ struct LdsRk4 : LdsEnv<TX, TY, TZ, FI, LdsRk4<STAGE, TX, TY, TZ, FI, FO, AX, DEF
                 Rk4SinkT<STAGE, FI, FO, AX, BufIo> {
   using Sink = Rk4SinkT<STAGE, FI, FO, AX, BufIo>;
   static constexpr bool kDefer = DEFER && STAGE < 3;
+  // the single-patch kernel's correctors issue both tiles late: sub-steps 1-3
+  // of 128^3 points 951 / 921 / 779 -> 927 / 899 / 770 us, but sub-step 0 with
+  // the residuals 1,066 -> 1,151
+  static constexpr int kDmaAt = DEFER && STAGE > 0 ? 2 : 1;
   int dv = -1;
   double dacc, dout;
   __device__ __forceinline__ void sink_rotate() { Sink::rotate(); }

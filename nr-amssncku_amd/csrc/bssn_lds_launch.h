@@ -6,46 +6,58 @@
 
 namespace amss {
 
-// 8-deep tiles (512 threads, one workgroup per CU) re-read less halo, 4-deep
-// ones (256 threads, two per CU) spread a small box over more CUs and end it
-// sooner.  The line is two rounds of 8-deep tiles on the chip's 256 CUs: per
-// sub-step of n^3 points, 4- against 8-deep, 32 against 42 us at 16^3, 37
-// against 46 at 32^3, 92 against 103 at 56^3 (343 tiles), 132 against 139 at
-// 64^3 (512), 526 against 496 at 96^3 (1728).
-inline int lds_tile_depth(const Box& box) {
-  long n8 = 1;
-  for (int a = 0; a < 3; ++a) n8 *= (box.hi[a] - box.lo[a] + 7) / 8;
-  return box.hi[2] - box.lo[2] >= 8 && n8 > 512 ? 8 : kLdsTZ;
+// The tile shape for an interior box.  4-deep 8x8 tiles (256 threads, two
+// workgroups per CU) spread a small box over more CUs and end it sooner: up to
+// two rounds of 512-point tiles on the chip's 256 CUs (per sub-step of n^3
+// points against 8x8x8, 32 against 42 us at 16^3, 37 against 46 at 32^3, 92
+// against 103 at 56^3 with 343 tiles, 132 against 139 at 64^3 with 512; the
+// other way 526 against 496 at 96^3 with 1728).  Above, rows of 32 points where
+// the box does not pad them away: their loads and stores touch whole cache
+// lines (an 8-point row of an array whose rows are not 64-byte aligned touches
+// two, half of each), which is worth more than the smaller halo of a cube:
+// sub-steps 0-3 of 128^3 points take 1,070 / 921 / 894 / 762 us against 1,230 /
+// 1,138 / 1,102 / 927, 0.84 of the time per point on average, so a 32x4x4 cover
+// may hold 1/0.84 of the cubic one's points.
+inline int lds_tile_shape(const Box& box) {
+  long n[3];  // points the cover by each shape computes
+  for (int s = 0; s < 3; ++s) {
+    n[s] = 1;
+    for (int a = 0; a < 3; ++a) n[s] *= (box.hi[a] - box.lo[a] + kLdsShape[s][a] - 1) / kLdsShape[s][a] * kLdsShape[s][a];
+  }
+  if (box.hi[2] - box.lo[2] < 8 || n[1] <= 512 * 512) return 0;
+  return n[2] * 0.84 < n[1] ? 2 : 1;
 }
 
 template <int G, bool ODD>
 void launch_rk4_lds(const FieldsIn& in, const FieldsIn& u0, const FieldsOut& acc, const FieldsOut& out,
                     const AuxOut& aux, const Box& box, const Coef& C, const Rk4Param& R, bool want_res, int* flag,
                     hipStream_t s) {
-  const int tz = lds_tile_depth(box);
-  const int nt = kLdsTX * kLdsTY * tz;
-  const int T[3] = {kLdsTX, kLdsTY, tz};
+  const int sh = lds_tile_shape(box);
+  const int* T = kLdsShape[sh];
+  const int nt = T[0] * T[1] * T[2];
   unsigned ntile = 1;
   for (int a = 0; a < 3; ++a) ntile *= (unsigned)((box.hi[a] - box.lo[a] + T[a] - 1) / T[a]);
   // the fused frozen-ghost fill (none unless rk4_fuses_fill)
   const long nfill = rk4_fuses_fill(box, R) ? ghost3_count(box.n[0], box.n[1], box.n[2]) : 0;
   const unsigned gr = ntile + (unsigned)((nfill + nt - 1) / nt);
-#define AMSS_LDS_ST(ST, CO, TZ) \
-  rk4_lds_kernel<G, ST, CO, TZ, ODD><<<gr, nt, 0, s>>>(in, u0, acc, out, aux, box, C, R, flag, nfill)
-#define AMSS_LDS(TZ)                           \
+#define AMSS_LDS_ST(ST, CO, SH) \
+  rk4_lds_kernel<G, ST, CO, SH, ODD><<<gr, nt, 0, s>>>(in, u0, acc, out, aux, box, C, R, flag, nfill)
+#define AMSS_LDS(SH)                           \
   switch (R.stage) {                           \
     case 0:                                    \
-      if (want_res) AMSS_LDS_ST(0, true, TZ);  \
-      else AMSS_LDS_ST(0, false, TZ);          \
+      if (want_res) AMSS_LDS_ST(0, true, SH);  \
+      else AMSS_LDS_ST(0, false, SH);          \
       break;                                   \
-    case 1: AMSS_LDS_ST(1, false, TZ); break;  \
-    case 2: AMSS_LDS_ST(2, false, TZ); break;  \
-    default: AMSS_LDS_ST(3, false, TZ); break; \
+    case 1: AMSS_LDS_ST(1, false, SH); break;  \
+    case 2: AMSS_LDS_ST(2, false, SH); break;  \
+    default: AMSS_LDS_ST(3, false, SH); break; \
   }
-  if (tz == 8) {
-    AMSS_LDS(8)
+  if (sh == 0) {
+    AMSS_LDS(0)
+  } else if (sh == 1) {
+    AMSS_LDS(1)
   } else {
-    AMSS_LDS(4)
+    AMSS_LDS(2)
   }
 #undef AMSS_LDS
 #undef AMSS_LDS_ST

@@ -2,7 +2,8 @@
 oracle at every point: axes shorter than a tile, one point past whole tiles,
 odd row and plane pitches (each parity has its own LDS layout; with an odd
 point count every other field starts off 16-byte alignment), and boxes on
-both sides of the tile-depth rule; per patch and batched.  Tolerance 1e-12 of
+both sides of the tile-shape rule (8x8x4, 8x8x8 and 32x4x4, each pitch); per
+patch and batched.  Tolerance 1e-12 of
 each field's largest value: one step's rounding, as in the other step tests."""
 import numpy as np
 import pytest
@@ -12,7 +13,7 @@ from helpers import NF, random_state, rel_err
 pytestmark = pytest.mark.gpu
 
 SHAPES = [(7, 7, 7), (8, 7, 9), (9, 8, 7), (14, 14, 14), (15, 14, 15), (15, 15, 15), (16, 23, 11), (23, 17, 22),
-          (22, 15, 31), (13, 40, 10), (70, 70, 71), (71, 71, 72)]
+          (22, 15, 31), (13, 40, 10), (70, 70, 71), (71, 71, 72), (78, 78, 71), (77, 77, 71)]
 
 
 @pytest.mark.parametrize("shape,gauge", [(s, 0) for s in SHAPES] + [(s, 2) for s in SHAPES if max(s) < 60])
