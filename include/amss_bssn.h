@@ -373,7 +373,7 @@ int amss_amr_checkpoint_write(amss_amr *A, const char *path, int movls, int nbh,
 int amss_amr_checkpoint_read(amss_amr *A, const char *path, int *movls, int *nbh, double *porg, int maxbh);
 /* Interior kernel of the fused RHS + RK4 sub-step: 0 reads every stencil
  * point through the vector L1/L2 (raw buffer loads); 1 stages a halo tile of
- * each field group in LDS (8x8x4-point tiles, double-buffered, filled by
+ * each field group in LDS (8x8x4 to 32x4x4-point tiles, double-buffered, filled by
  * direct global->LDS loads; the default).  Both give the same results to
  * rounding. */
 int amss_level_set_variant(amss_level *L, int variant);
@@ -385,7 +385,8 @@ int amss_level_variant(amss_level *L);
 int amss_level_timing(amss_level *L, int enable);
 int amss_level_kernel_ms(amss_level *L, double *ms4, long *launches4);
 /* Batched step (modes 1, 2): the interior of every patch is cut into tiles of
- * one of AMSS_NUM_TILE_SHAPES shapes (0: 8x8x4, 1: 4x8x8, 2: 8x4x8, 3: 8x8x8 points);
+ * one of AMSS_NUM_TILE_SHAPES shapes (0: 8x8x4, 1: 4x8x8, 2: 8x4x8, 3: 8x8x8 points,
+ * with 32x4x4 tiles along x as far as they fit);
  * one launch per sub-step walks the tile list of all patches with `grid`
  * persistent workgroups (0: one workgroup per tile), in list order or
  * (remap 1) with each XCD given a contiguous run of tiles.  autotune times

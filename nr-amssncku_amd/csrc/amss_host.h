@@ -179,11 +179,12 @@ class BssnLevel {
   std::vector<Ev> ev_;       // event pairs of the current step() call
   size_t ev_used_ = 0;
   // batched step: device tables of patches, tiles (per tile shape), boundary
-  // boxes and exchange boxes; interior remainders that no whole tile covers
+  // boxes and exchange boxes; patches launched one by one (odd row pitches)
   std::vector<PatchDesc> hpd_;
   PatchDesc* dpd_ = nullptr;
   std::vector<TileRef> htiles_[kNumTileShapes];
   TileRef* dtiles_[kNumTileShapes] = {};
+  int nwide_[kNumTileShapes] = {};  // 32x4x4 tiles at the start of the list (shape 3)
   std::vector<std::pair<int, Box>> rem_[kNumTileShapes];
   // ghost boxes (fill boxes, then exchange boxes) and their work list: fill
   // entries [0, nfill_work_), exchange entries after them

@@ -553,6 +553,7 @@ void BssnLevel::build_batch_tables() {
   LCHK(hipMemcpy(dpd_, hpd_.data(), np * sizeof(PatchDesc), hipMemcpyHostToDevice));
   for (int sh = 0; sh < kNumTileShapes; ++sh) {
     const int T[3] = {tile_dim(sh, 0), tile_dim(sh, 1), tile_dim(sh, 2)};
+    std::vector<TileRef> wide;  // before the others in the list
     htiles_[sh].clear();
     rem_[sh].clear();
     for (int pi = 0; pi < np; ++pi) {
@@ -583,12 +584,24 @@ void BssnLevel::build_batch_tables() {
         return;
       }
       // whole and partial tiles: the kernel masks the points past the interior
+      auto add = [&](std::vector<TileRef>& to, int i, int j, int k) {
+        to.push_back(TileRef{(unsigned short)pi, (unsigned short)i, (unsigned short)j, (unsigned short)k});
+      };
+      int x0 = 3;  // 32x4x4 tiles on [3, x0), in strips of 4 x 4 points along y
+      if (sh == 3) {
+        while (box.hi[0] - x0 >= kWideFill) x0 += kWideX;
+        x0 = std::min(x0, box.hi[0]);
+        for (int js = 3; x0 > 3 && js < box.hi[1]; js += 4 * kWideYZ)
+          for (int k = 3; k < box.hi[2]; k += kWideYZ)
+            for (int j = js; j < std::min(js + 4 * kWideYZ, box.hi[1]); j += kWideYZ)
+              for (int i = 3; i < x0; i += kWideX) add(wide, i, j, k);
+      }
       for (int k = 3; k < box.hi[2]; k += T[2])
         for (int j = 3; j < box.hi[1]; j += T[1])
-          for (int i = 3; i < box.hi[0]; i += T[0])
-            htiles_[sh].push_back(TileRef{(unsigned short)pi, (unsigned short)i, (unsigned short)j,
-                                          (unsigned short)k});
+          for (int i = x0; i < box.hi[0]; i += T[0]) add(htiles_[sh], i, j, k);
     }
+    nwide_[sh] = (int)wide.size();
+    htiles_[sh].insert(htiles_[sh].begin(), wide.begin(), wide.end());
     if ((long)htiles_[sh].size() > (1L << 31) - 1) { err_ = "too many tiles"; return; }
     if (!htiles_[sh].empty()) {
       LCHK(hipMalloc(&dtiles_[sh], htiles_[sh].size() * sizeof(TileRef)));
@@ -717,12 +730,12 @@ int BssnLevel::StepBatched(double dT, bool want_res) {
     // With frozen ghosts the fill reads only the state and writes only
     // points no tile writes: it runs in extra workgroups of the tile launch.
     const int ntiles = (int)htiles_[sh].size();
-    const bool fill_in_tiles = frozen && ghost_fused_ && launch_rk4_tiles_fuses_fill(tune_, ntiles);
+    const bool fill_in_tiles = frozen && ghost_fused_ && launch_rk4_tiles_fuses_fill(tune_, ntiles, nwide_[sh]);
     FillWork fw;
     if (fill_in_tiles && fill) fw = FillWork{dgbox_, dgwork_, nfill_work_};
     Ev* ev = nullptr;
     if (int r = time_event_begin(it, &ev)) return r;
-    launch_rk4_tiles(gauge_, dpd_, dtiles_[sh], 0, ntiles, m, coef_[0], R, res, tune_, dflag_, stream_, fw);
+    launch_rk4_tiles(gauge_, dpd_, dtiles_[sh], ntiles, nwide_[sh], m, coef_[0], R, res, tune_, dflag_, stream_, fw);
     if (ev) RCHK(hipEventRecord(ev->b, stream_));
     AuxOut aux;
     for (int a = 0; a < 18; ++a) aux.gam[a] = nullptr;
@@ -846,8 +859,8 @@ int BssnLevel::autotune(double* ms, int nms) {
         float tbest = 1e30f;
         for (int rep = 0; rep < 3; ++rep) {
           RCHK(hipEventRecord(e0, stream_));
-          launch_rk4_tiles(gauge_, dpd_, dtiles_[sh], 0, (int)htiles_[sh].size(), m, coef_[0], R, false, t, dflag_,
-                           stream_);
+          launch_rk4_tiles(gauge_, dpd_, dtiles_[sh], (int)htiles_[sh].size(), nwide_[sh], m, coef_[0], R, false, t,
+                           dflag_, stream_);
           for (const auto& pr : rem_[sh]) {
             const Block& b = *blocks_[pr.first];
             for (int a = 0; a < 7; ++a) aux.res[a] = b.fgfs[kResidualBase + a];

@@ -90,10 +90,16 @@ struct FillWork {
   int n = 0;  // 256-point work items
 };
 
-// Tile shapes of the batched kernel (points per tile along x, y, z).
+// Tile shapes of the batched kernel (points per tile along x, y, z).  Shape 3
+// is 512 points, two launches: 32x4x4 along x while whole tiles fit (or one
+// full to kWideFill points), then 8x8x8 for the rest of the rows.  A 32-point
+// row touches whole cache lines where an 8-point one straddles two
+// (lds_tile_shape has the figures).  Both in one launch, a branch per tile, cost
+// 60 bytes of scratch per lane: 37 patches 21.1 ms against 20.5.
+constexpr int kWideX = 32, kWideYZ = 4, kWideFill = 27;
 constexpr int kNumTileShapes = 4;
 __host__ __device__ constexpr int tile_dim(int shape, int a) {
-  // 0: 8x8x4, 1: 4x8x8, 2: 8x4x8 (256 threads); 3: 8x8x8 (512 threads)
+  // 0: 8x8x4, 1: 4x8x8, 2: 8x4x8 (256 threads); 3: 8x8x8 (and 32x4x4; 512 threads)
   return shape == 0 ? (a == 2 ? 4 : 8) : shape == 1 ? (a == 0 ? 4 : 8) : shape == 2 ? (a == 1 ? 4 : 8) : 8;
 }
 
@@ -111,18 +117,20 @@ struct BatchTune {
   int remap;   // 1 = XCD-contiguous tile order
 };
 
-// Fused RHS + RK4 sub-step over tiles [t0, t0 + ntiles) of the tile list.
-// fw: fill work run in extra workgroups (only with one workgroup per tile:
-// launch_rk4_tiles_fuses_fill).
-void launch_rk4_tiles(int gauge, const PatchDesc* P, const TileRef* T, int t0, int ntiles, const Roles& m,
+// Fused RHS + RK4 sub-step over the ntiles tiles of the list T, the first
+// nwide of them 32x4x4 (shape 3 only).
+// fw: fill work run in extra workgroups of the last launch (only with one
+// workgroup per tile there: launch_rk4_tiles_fuses_fill).
+void launch_rk4_tiles(int gauge, const PatchDesc* P, const TileRef* T, int ntiles, int nwide, const Roles& m,
                       const Coef& C, const Rk4Param& R, bool want_res, const BatchTune& tune, int* flag,
                       hipStream_t s, const FillWork& fw = FillWork{});
-inline bool launch_rk4_tiles_fuses_fill(const BatchTune& tune, int ntiles) {
-  return !(tune.grid > 0 && tune.grid < ntiles) && ntiles > 0;
+inline bool launch_rk4_tiles_fuses_fill(const BatchTune& tune, int ntiles, int nwide) {
+  const int last = ntiles > nwide ? ntiles - nwide : nwide;
+  return !(tune.grid > 0 && tune.grid < last) && ntiles > 0;
 }
-#define AMSS_DECL_TILES(G, S)                                                                             \
-  void launch_rk4_tiles_g##G##_s##S(const PatchDesc* P, const TileRef* T, int t0, int ntiles, const Roles& m, \
-                                    const Coef& C, const Rk4Param& R, bool want_res, const BatchTune& tune,  \
+#define AMSS_DECL_TILES(G, S)                                                                                  \
+  void launch_rk4_tiles_g##G##_s##S(const PatchDesc* P, const TileRef* T, int ntiles, int nwide, const Roles& m, \
+                                    const Coef& C, const Rk4Param& R, bool want_res, const BatchTune& tune,    \
                                     int* flag, hipStream_t s, const FillWork& fw);
 AMSS_DECL_TILES(0, 0)
 AMSS_DECL_TILES(0, 1)

@@ -114,12 +114,12 @@ unsigned xblocks(long maxpts) {
 
 }  // namespace
 
-void launch_rk4_tiles(int gauge, const PatchDesc* P, const TileRef* T, int t0, int ntiles, const Roles& m,
+void launch_rk4_tiles(int gauge, const PatchDesc* P, const TileRef* T, int ntiles, int nwide, const Roles& m,
                       const Coef& C, const Rk4Param& R, bool want_res, const BatchTune& tune, int* flag,
                       hipStream_t s, const FillWork& fw) {
 #define AMSS_CASE(G, S)                                                                      \
   case S:                                                                                    \
-    launch_rk4_tiles_g##G##_s##S(P, T, t0, ntiles, m, C, R, want_res, tune, flag, s, fw); \
+    launch_rk4_tiles_g##G##_s##S(P, T, ntiles, nwide, m, C, R, want_res, tune, flag, s, fw); \
     break;
   if (gauge == 2) {
     switch (tune.shape) { AMSS_CASE(2, 0) AMSS_CASE(2, 1) AMSS_CASE(2, 2) AMSS_CASE(2, 3) }

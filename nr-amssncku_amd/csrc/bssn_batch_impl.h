@@ -43,7 +43,7 @@ __device__ __forceinline__ void tile_body(const PatchDesc* __restrict__ P, const
 // iterations and spill more).
 template <int GAUGE, int STAGE, bool CO, int TX, int TY, int TZ, bool PERSIST>
 __global__ void __launch_bounds__(TX* TY* TZ) __attribute__((amdgpu_waves_per_eu(2, 2)))
-rk4_tiles_kernel(const PatchDesc* __restrict__ P, const TileRef* __restrict__ T, int t0, int ntiles, Roles m,
+rk4_tiles_kernel(const PatchDesc* __restrict__ P, const TileRef* __restrict__ T, int ntiles, Roles m,
                  Coef C, Rk4Param R, int remap, int* flag, FillWork fw) {
   using Tl = LdsTile<TX, TY, TZ>;
   __shared__ __attribute__((aligned(16))) double tiles[kLdsBuffers * Tl::NPAD];
@@ -61,23 +61,22 @@ rk4_tiles_kernel(const PatchDesc* __restrict__ P, const TileRef* __restrict__ T,
       // loop (hundreds of loop-invariant addresses would occupy VGPRs)
       int tid = threadIdx.x;
       asm volatile("" : "+v"(tid));
-      const TileRef r = T[t0 + (remap ? xcd_spread(t, ntiles) : t)];
+      const TileRef r = T[remap ? xcd_spread(t, ntiles) : t];
       tile_body<GAUGE, STAGE, CO, TX, TY, TZ>(P, r, m, C, R, flag, b0, tid);
     }
   } else {
     const int t = blockIdx.x;
-    const TileRef r = T[t0 + (remap ? xcd_spread(t, ntiles) : t)];
+    const TileRef r = T[remap ? xcd_spread(t, ntiles) : t];
     tile_body<GAUGE, STAGE, CO, TX, TY, TZ>(P, r, m, C, R, flag, b0, (int)threadIdx.x);
   }
 }
 
 template <int G, int TX, int TY, int TZ, bool PERSIST>
-void launch_tiles_p(unsigned g, const PatchDesc* P, const TileRef* T, int t0, int ntiles, const Roles& m,
-                    const Coef& C, const Rk4Param& R, bool want_res, int remap, int* flag, hipStream_t s,
-                    const FillWork& fw) {
+void launch_tiles_p(unsigned g, const PatchDesc* P, const TileRef* T, int ntiles, const Roles& m, const Coef& C,
+                    const Rk4Param& R, bool want_res, int remap, int* flag, hipStream_t s, const FillWork& fw) {
   const int nt = TX * TY * TZ;
 #define AMSS_TILES(ST, CO) \
-  rk4_tiles_kernel<G, ST, CO, TX, TY, TZ, PERSIST><<<g, nt, 0, s>>>(P, T, t0, ntiles, m, C, R, remap, flag, fw)
+  rk4_tiles_kernel<G, ST, CO, TX, TY, TZ, PERSIST><<<g, nt, 0, s>>>(P, T, ntiles, m, C, R, remap, flag, fw)
   switch (R.stage) {
     case 0:
       if (want_res) AMSS_TILES(0, true);
@@ -90,31 +89,43 @@ void launch_tiles_p(unsigned g, const PatchDesc* P, const TileRef* T, int t0, in
 #undef AMSS_TILES
 }
 
-// Fill work rides along only with one workgroup per tile (the caller runs it
-// separately otherwise: launch_rk4_tiles_fuses_fill).
+// Tiles of one shape.  Fill work rides along only with one workgroup per tile
+// (the caller runs it separately otherwise: launch_rk4_tiles_fuses_fill).
 template <int G, int TX, int TY, int TZ>
-void launch_rk4_tiles_shape(const PatchDesc* P, const TileRef* T, int t0, int ntiles, const Roles& m,
-                            const Coef& C, const Rk4Param& R, bool want_res, const BatchTune& tune, int* flag,
-                            hipStream_t s, const FillWork& fw) {
-  if (ntiles <= 0) return;
+void launch_rk4_tiles_of(const PatchDesc* P, const TileRef* T, int ntiles, const Roles& m, const Coef& C,
+                         const Rk4Param& R, bool want_res, const BatchTune& tune, int* flag, hipStream_t s,
+                         const FillWork& fw) {
   constexpr int kItems = TX * TY * TZ / 256;
   if (tune.grid > 0 && tune.grid < ntiles) {
-    launch_tiles_p<G, TX, TY, TZ, true>((unsigned)tune.grid, P, T, t0, ntiles, m, C, R, want_res, tune.remap, flag, s,
+    launch_tiles_p<G, TX, TY, TZ, true>((unsigned)tune.grid, P, T, ntiles, m, C, R, want_res, tune.remap, flag, s,
                                         FillWork{});
   } else {
     const unsigned extra = (unsigned)((fw.n + kItems - 1) / kItems);
-    launch_tiles_p<G, TX, TY, TZ, false>((unsigned)ntiles + extra, P, T, t0, ntiles, m, C, R, want_res, tune.remap,
-                                         flag, s, fw);
+    launch_tiles_p<G, TX, TY, TZ, false>((unsigned)ntiles + extra, P, T, ntiles, m, C, R, want_res, tune.remap, flag,
+                                         s, fw);
   }
 }
 
+template <int G, int TX, int TY, int TZ>
+void launch_rk4_tiles_shape(const PatchDesc* P, const TileRef* T, int ntiles, int nwide, const Roles& m, const Coef& C,
+                            const Rk4Param& R, bool want_res, const BatchTune& tune, int* flag, hipStream_t s,
+                            const FillWork& fw) {
+  if constexpr (TX * TY * TZ == kWideX * kWideYZ * kWideYZ) {
+    if (nwide > 0)
+      launch_rk4_tiles_of<G, kWideX, kWideYZ, kWideYZ>(P, T, nwide, m, C, R, want_res, tune, flag, s,
+                                                       ntiles > nwide ? FillWork{} : fw);
+  }
+  if (ntiles > nwide)
+    launch_rk4_tiles_of<G, TX, TY, TZ>(P, T + nwide, ntiles - nwide, m, C, R, want_res, tune, flag, s, fw);
+}
+
 // One translation unit per gauge and tile shape (they compile in parallel).
-#define AMSS_BATCH_TU(G, S)                                                                                  \
-  void launch_rk4_tiles_g##G##_s##S(const PatchDesc* P, const TileRef* T, int t0, int ntiles, const Roles& m, \
-                                    const Coef& C, const Rk4Param& R, bool want_res, const BatchTune& tune,  \
-                                    int* flag, hipStream_t s, const FillWork& fw) {                          \
-    launch_rk4_tiles_shape<G, tile_dim(S, 0), tile_dim(S, 1), tile_dim(S, 2)>(P, T, t0, ntiles, m, C, R,      \
-                                                                              want_res, tune, flag, s, fw);  \
+#define AMSS_BATCH_TU(G, S)                                                                                      \
+  void launch_rk4_tiles_g##G##_s##S(const PatchDesc* P, const TileRef* T, int ntiles, int nwide, const Roles& m,  \
+                                    const Coef& C, const Rk4Param& R, bool want_res, const BatchTune& tune,      \
+                                    int* flag, hipStream_t s, const FillWork& fw) {                              \
+    launch_rk4_tiles_shape<G, tile_dim(S, 0), tile_dim(S, 1), tile_dim(S, 2)>(P, T, ntiles, nwide, m, C, R,       \
+                                                                              want_res, tune, flag, s, fw);      \
   }
 
 }  // namespace amss

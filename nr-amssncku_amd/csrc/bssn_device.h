@@ -52,11 +52,18 @@ struct FieldsOut {
 typedef __attribute__((address_space(1))) double gdouble;
 
 // The 24 fields of one time level inside a Block's slab: field v starts at
-// base + v * n (a Block keeps its lists as consecutive 24-field runs).
+// base + v * n (a Block keeps its lists as consecutive 24-field runs).  The
+// empty asm has each address formed where it is used: kept instead, the
+// products v * n spilled some 60 scalar registers of the tile-list kernels and
+// with them 40 bytes per lane (37 patches, sub-step 1: 4.41 -> 4.26 ms).
 struct SlabFields {
   gdouble* base;
   long n;
-  __device__ __forceinline__ gdouble* ptr(int v) const { return base + v * n; }
+  __device__ __forceinline__ gdouble* ptr(int v) const {
+    long m = n;
+    asm volatile("" : "+s"(m));
+    return base + v * m;
+  }
 };
 
 // Finite-difference coefficients of one patch (host-computed from

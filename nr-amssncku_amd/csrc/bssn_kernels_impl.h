@@ -204,7 +204,7 @@ rk4_lds_kernel(FieldsIn in, FieldsIn u0, FieldsOut acc, FieldsOut out, AuxOut au
   bool live;
   const BufIo io = tile_io(i0 + tx, j0 + ty, k0 + tz, box.hi[0], box.hi[1], box.hi[2], (int)box.sy, (int)box.sz, N, live);
   lds_double* t0 = (lds_double*)tiles;
-  LdsRk4<STAGE, TX, TY, TZ, FieldsIn, FieldsOut, AuxOut, true, ODD> X{
+  LdsRk4<STAGE, TX, TY, TZ, FieldsIn, FieldsOut, AuxOut, ODD, (STAGE > 0 ? 2 : 1)> X{
       {in, in, C, t0, t0 + (kLdsBuffers / 2) * Tl::NPAD, io, Tl::lds_index(tx, ty, tz, (int)box.sz),
        (int)((i0 - 3) + (j0 - 3) * box.sy + (k0 - 3) * box.sz), (int)box.sy, (int)box.sz, N, (int)threadIdx.x, tz + 3},
       {u0, acc, out, aux, io, R.c, R.tinny, {}}};

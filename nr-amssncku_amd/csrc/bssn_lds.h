@@ -343,23 +343,23 @@ struct LdsEnv {
 
 // The LDS environment and the RK4 epilogue as one object (passed to the point
 // algebra as both), so the environment can hand the epilogue its prefetches.
-// DEFER: the last put's stores wait for the next group boundary, where the
-// environment calls sink_flush after its barrier -- a store issued just
-// before a barrier would be waited for there (its s_waitcnt(0) waits for
-// every memory operation), one issued after it has a group's computation to
-// land.  Measured on one box against the immediate stores: the single-patch
-// kernel +0.9%, the tile-list kernel -1.4%, so only the former defers; and
-// sub-step 3, one store per field, gains nothing.
+// The last put's stores wait for the next group boundary, where the
+// environment calls sink_flush after its barrier -- a store issued just before
+// a barrier would be waited for there (its s_waitcnt(0) waits for every memory
+// operation), one issued after it has a group's computation to land: 37
+// patches 20.63 -> 20.47 ms, 128^3 +0.9%.  Sub-step 3, one store per field,
+// gains nothing.
+// DMA: when the halo tiles are issued (DmaAt).  The single-patch kernel's
+// correctors issue both late: sub-steps 1-3 of 128^3 points 951 / 921 / 779 ->
+// 927 / 899 / 770 us; sub-step 0 with the residuals loses by it (1,066 ->
+// 1,151), and so do the tile lists (18.1 -> 18.3 ms).
 template <int STAGE, int TX, int TY, int TZ, class FI = FieldsIn, class FO = FieldsOut, class AX = AuxOut,
-          bool DEFER = false, bool ODD = false>
-struct LdsRk4 : LdsEnv<TX, TY, TZ, FI, LdsRk4<STAGE, TX, TY, TZ, FI, FO, AX, DEFER, ODD>, ODD>,
+          bool ODD = false, int DMA = 1>
+struct LdsRk4 : LdsEnv<TX, TY, TZ, FI, LdsRk4<STAGE, TX, TY, TZ, FI, FO, AX, ODD, DMA>, ODD>,
                 Rk4SinkT<STAGE, FI, FO, AX, BufIo> {
   using Sink = Rk4SinkT<STAGE, FI, FO, AX, BufIo>;
-  static constexpr bool kDefer = DEFER && STAGE < 3;
-  // the single-patch kernel's correctors issue both tiles late: sub-steps 1-3
-  // of 128^3 points 951 / 921 / 779 -> 927 / 899 / 770 us, but sub-step 0 with
-  // the residuals 1,066 -> 1,151
-  static constexpr int kDmaAt = DEFER && STAGE > 0 ? 2 : 1;
+  static constexpr bool kDefer = STAGE < 3;
+  static constexpr int kDmaAt = DMA;
   int dv = -1;
   double dacc, dout;
   __device__ __forceinline__ void sink_rotate() { Sink::rotate(); }
