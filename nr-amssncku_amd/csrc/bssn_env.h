@@ -338,25 +338,29 @@ struct PtrIo {
 // nothing: the hardware drops buffer stores at or past the buffer's end, so
 // the point kernels mask their stores without a branch.  (Shared 32-bit
 // offsets also took the tile-list step of 37 patches from 22.8 to 21.8 ms.)
+// NTL, NTS: loads / stores marked non-temporal (LdsRk4, bssn_lds.h).
 constexpr unsigned kDropStore = 0xFFFFFFF8u;  // >= bytes of any array (at most 2^29 - 1 points)
-struct BufIo {
+template <bool NTL = false, bool NTS = false>
+struct BufIoT {
   unsigned vo;     // byte offset of the point (clamped into the interior)
   unsigned vs;     // vo, or kDropStore
   unsigned bytes;  // of one array
+  static constexpr int kNt = 2;  // the nt bit of a buffer instruction's cache policy
   template <class P>
   __device__ __forceinline__ __amdgpu_buffer_rsrc_t rsrc(P a) const {
     return __builtin_amdgcn_make_buffer_rsrc((void*)a, (short)0, (int)bytes, 0x00020000);
   }
   template <class P>
   __device__ __forceinline__ double ld(P a) const {
-    return __builtin_bit_cast(double, __builtin_amdgcn_raw_buffer_load_b64(rsrc(a), vo, 0, 0));
+    return __builtin_bit_cast(double, __builtin_amdgcn_raw_buffer_load_b64(rsrc(a), vo, 0, NTL ? kNt : 0));
   }
   template <class P>
   __device__ __forceinline__ void st(P a, double x) const {
     typedef unsigned v2u __attribute__((ext_vector_type(2)));
-    __builtin_amdgcn_raw_buffer_store_b64(__builtin_bit_cast(v2u, x), rsrc(a), vs, 0, 0);
+    __builtin_amdgcn_raw_buffer_store_b64(__builtin_bit_cast(v2u, x), rsrc(a), vs, 0, NTS ? kNt : 0);
   }
 };
+using BufIo = BufIoT<>;
 
 // RK4 sub-step sink (rungekutta4_rout.f90:110-128 fused into the RHS
 // epilogue), followed by the lower bound on chi (fmisc.f90:1644-1657) and,

@@ -177,7 +177,7 @@ rk4_lds_kernel(FieldsIn in, FieldsIn u0, FieldsOut acc, FieldsOut out, AuxOut au
                                  Coef C, Rk4Param R, int* flag, long nfill) {
   constexpr int TX = kLdsShape[SH][0], TY = kLdsShape[SH][1], TZ = kLdsShape[SH][2];
   using Tl = LdsTile<TX, TY, TZ, ODD>;
-  __shared__ __attribute__((aligned(16))) double tiles[kLdsBuffers * Tl::NPAD];
+  __shared__ __attribute__((aligned(16))) double tiles[kLdsBuffers * Tl::NPAD + lds_stash(TX * TY * TZ, Tl::NPAD)];
   const int gx = (box.hi[0] - box.lo[0] + TX - 1) / TX, gy = (box.hi[1] - box.lo[1] + TY - 1) / TY;
   const int gz = (box.hi[2] - box.lo[2] + TZ - 1) / TZ, ntiles = gx * gy * gz;
   if ((int)blockIdx.x >= ntiles) {
@@ -204,10 +204,12 @@ rk4_lds_kernel(FieldsIn in, FieldsIn u0, FieldsOut acc, FieldsOut out, AuxOut au
   bool live;
   const BufIo io = tile_io(i0 + tx, j0 + ty, k0 + tz, box.hi[0], box.hi[1], box.hi[2], (int)box.sy, (int)box.sz, N, live);
   lds_double* t0 = (lds_double*)tiles;
-  LdsRk4<STAGE, TX, TY, TZ, FieldsIn, FieldsOut, AuxOut, ODD, (STAGE > 0 ? 2 : 1)> X{
+  using Rk = LdsRk4<STAGE, TX, TY, TZ, FieldsIn, FieldsOut, AuxOut, ODD, (STAGE > 0 ? 2 : 1), SH == 2>;
+  Rk X{
       {in, in, C, t0, t0 + (kLdsBuffers / 2) * Tl::NPAD, io, Tl::lds_index(tx, ty, tz, (int)box.sz),
        (int)((i0 - 3) + (j0 - 3) * box.sy + (k0 - 3) * box.sz), (int)box.sy, (int)box.sz, N, (int)threadIdx.x, tz + 3},
-      {u0, acc, out, aux, io, R.c, R.tinny, {}}};
+      {u0, acc, out, aux, typename Rk::Io{io.vo, io.vs, io.bytes}, R.c, R.tinny, {}},
+       t0 + kLdsBuffers * Tl::NPAD + threadIdx.x};
   X.prologue();
   bssn_rhs_point<GAUGE, CO, false, false>(X, X);
   X.finish();

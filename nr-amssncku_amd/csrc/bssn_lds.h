@@ -112,6 +112,14 @@ __device__ __forceinline__ BufIo tile_io(int i, int j, int k, int hx, int hy, in
 // or two single buffers.
 constexpr int kLdsBuffers = AMSS_LDS_PAIRS ? 4 : 2;
 
+// Doubles of the epilogue's stash (LdsRk4) behind a kernel's tile buffers of
+// npad doubles each, for workgroups of `points` threads: 6 per thread, or none
+// where the workgroups of one CU (2 waves per SIMD: 512 threads) would then
+// not fit its 160 KB (the 8x8x4 tiles of odd pitches).
+constexpr int lds_stash(int points, int npad) {
+  return (512 / points) * (kLdsBuffers * npad + 6 * points) * 8 <= 160 * 1024 ? 6 * points : 0;
+}
+
 #ifndef AMSS_TOP
 #define AMSS_TOP 1
 #endif
@@ -353,13 +361,29 @@ struct LdsEnv {
 // correctors issue both late: sub-steps 1-3 of 128^3 points 951 / 921 / 779 ->
 // 927 / 899 / 770 us; sub-step 0 with the residuals loses by it (1,066 ->
 // 1,151), and so do the tile lists (18.1 -> 18.3 ms).
+// Non-temporal traffic (WIDE_NT, wide tiles): what a sub-step writes, and what
+// a corrector reads of the old state and the accumulator, is not touched
+// again before the next sub-step, and wide tiles are used on boxes whose 24
+// fields exceed the caches; marked so, it leaves the L2 to the halo tiles.
+// The predictor's old state IS the field its halo tiles are filled from, so
+// its loads stay plain.  128^3 points, sub-steps 0-3 (residuals in 0):
+// 1081 / 932 / 906 / 768 -> 1014 / 916 / 892 / 764 us.  72^3 points on
+// 8x8x8 tiles lose 0.7% by it.
+// The six metric values that the epilogue keeps to the end wait in the
+// workgroup's spare LDS (STASH) instead of in registers, where the compiler
+// spilled them to scratch memory: 128^3 sub-steps 1 and 2 932 / 906 -> 893 / 869 us, 72^3
+// 215 / 201 -> 206 / 189.
 template <int STAGE, int TX, int TY, int TZ, class FI = FieldsIn, class FO = FieldsOut, class AX = AuxOut,
-          bool ODD = false, int DMA = 1>
-struct LdsRk4 : LdsEnv<TX, TY, TZ, FI, LdsRk4<STAGE, TX, TY, TZ, FI, FO, AX, ODD, DMA>, ODD>,
-                Rk4SinkT<STAGE, FI, FO, AX, BufIo> {
-  using Sink = Rk4SinkT<STAGE, FI, FO, AX, BufIo>;
+          bool ODD = false, int DMA = 1, bool WIDE_NT = false>
+struct LdsRk4 : LdsEnv<TX, TY, TZ, FI, LdsRk4<STAGE, TX, TY, TZ, FI, FO, AX, ODD, DMA, WIDE_NT>, ODD>,
+                Rk4SinkT<STAGE, FI, FO, AX, BufIoT<WIDE_NT && (STAGE > 0), WIDE_NT>> {
+  using Io = BufIoT<WIDE_NT && (STAGE > 0), WIDE_NT>;
+  using Sink = Rk4SinkT<STAGE, FI, FO, AX, Io>;
+  static constexpr int kPoints = TX * TY * TZ;
   static constexpr bool kDefer = STAGE < 3;
+  static constexpr bool kStash = STAGE < 3 && lds_stash(kPoints, LdsTile<TX, TY, TZ, ODD>::NPAD) > 0;
   static constexpr int kDmaAt = DMA;
+  lds_double* stash;  // this thread's first slot, slots kPoints apart (kStash)
   int dv = -1;
   double dacc, dout;
   __device__ __forceinline__ void sink_rotate() { Sink::rotate(); }
@@ -381,13 +405,19 @@ struct LdsRk4 : LdsEnv<TX, TY, TZ, FI, LdsRk4<STAGE, TX, TY, TZ, FI, FO, AX, ODD
     sink_flush();  // an earlier put since the last boundary
     dv = v;
     dacc = accv;
-    if (STAGE < 3 && v >= DXX && v <= AZZ)
+    if (kStash && v >= DXX && v <= DZZ)
+      stash[(v - DXX) * kPoints] = u;
+    else if (STAGE < 3 && v >= DXX && v <= AZZ)
       Sink::gA[v - DXX] = u;
     else
       dout = u;
   }
   __device__ __forceinline__ void finish() {
     sink_flush();
+    if (kStash) {
+#pragma unroll
+      for (int s = 0; s < 6; ++s) Sink::gA[s] = stash[s * kPoints];
+    }
     Sink::finish();
   }
 };
