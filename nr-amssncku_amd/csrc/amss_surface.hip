@@ -11,8 +11,24 @@ namespace amss {
 namespace {
 
 // global_interp's 6^3 block (cell-centred, decide3d's mirror below a
-// symmetry plane) of two fields at q, interpolated along z, y, x.
-__device__ void interp2(const SphereGrid& G, const double q[3], double out[2]) {
+// symmetry plane) of two fields at each sphere point, interpolated along z,
+// y, x: 43 tableaux of 15 dependent divisions per field.  A sphere has some
+// thousands of points, so one thread per point leaves the chip nearly empty
+// and its time is one thread's chain of 86 tableaux (12,800 points: 253 us).  Here a
+// point is 12 threads, one per field and x plane of the block, with 7 tableaux
+// each (neighbours in x read neighbouring elements); the last tableau, along
+// x, is the first of its field's six threads': 62 us, the same bits.
+constexpr int kSpherePer = 12, kSpherePoints = 20;  // threads per point; points per workgroup
+__global__ void __launch_bounds__(kSpherePer* kSpherePoints)
+sphere_interp_kernel(SphereGrid G, SphereRule R, double* __restrict__ vals) {
+  __shared__ double ym[kSpherePoints * kSpherePer];
+  const int tid = (int)threadIdx.x, a = tid % 6, f = tid / 6 % 2;
+  // (a last workgroup's threads past the end redo the last point, and store nothing)
+  const int np = R.n_theta * R.n_phi, want = blockIdx.x * kSpherePoints + tid / kSpherePer;
+  const int n = min(want, np - 1);
+  const int i = n / R.n_phi, j = n - i * R.n_phi;
+  const double ct = R.costheta[i], st = sqrt(1.0 - ct * ct), ph = (j + 0.5) * R.dphi;
+  const double q[3] = {R.rex * (st * cos(ph)), R.rex * (st * sin(ph)), R.rex * ct};
   const double* C[3] = {G.X, G.Y, G.Z};
   int cxB[3];
   double cx[3];
@@ -33,50 +49,37 @@ __device__ void interp2(const SphereGrid& G, const double q[3], double out[2]) {
     cxB[m] = b;
     cx[m] = b > 0 ? (q[m] - C[m][b - 1]) / d : (q[m] + C[m][-b]) / d;
   }
-  for (int f = 0; f < 2; ++f) {
-    const double* F = f == 0 ? G.rpsi : G.ipsi;
-    const double* S = f == 0 ? G.soa_r : G.soa_i;
-    double ym[6];
-    for (int a = 0; a < 6; ++a) {
-      double yz[6];
-      for (int b = 0; b < 6; ++b) {
-        double line[6];
+  const double* F = f == 0 ? G.rpsi : G.ipsi;
+  const long sy = G.n[0], sz = (long)G.n[0] * G.n[1];
+  // the mirrored index below a symmetry plane, and its sign
+  auto fold = [&](int m, int g, double& s) {
+    if (g >= 1) return g - 1;
+    s *= f == 0 ? G.soa_r[m] : G.soa_i[m];
+    return -g;
+  };
+  double sx = 1.0;
+  const int ix = fold(0, cxB[0] + a, sx);
+  double yz[6];
+  for (int b = 0; b < 6; ++b) {
+    double sxy = sx;
+    const long row = ix + fold(1, cxB[1] + b, sxy) * sy;
+    double line[6];
 #pragma unroll
-        for (int c = 0; c < 6; ++c) {
-          const int g[3] = {cxB[0] + a, cxB[1] + b, cxB[2] + c};
-          double s = 1.0;
-          long idx = 0;
-          const long st[3] = {1, G.n[0], (long)G.n[0] * G.n[1]};
-#pragma unroll
-          for (int m = 0; m < 3; ++m) {
-            int gi = g[m];
-            if (gi < 1) {
-              gi = 1 - gi;
-              s *= S[m];
-            }
-            idx += (gi - 1) * st[m];
-          }
-          const double v = F[idx];
-          line[c] = s == 1.0 ? v : v * s;
-        }
-        yz[b] = neville6(line, cx[2]);
-      }
-      ym[a] = neville6(yz, cx[1]);
+    for (int c = 0; c < 6; ++c) {
+      double s = sxy;
+      const double v = F[row + fold(2, cxB[2] + c, s) * sz];
+      line[c] = s == 1.0 ? v : v * s;
     }
-    out[f] = neville6(ym, cx[0]);
+    yz[b] = neville6(line, cx[2]);
   }
-}
-
-__global__ void __launch_bounds__(256) sphere_interp_kernel(SphereGrid G, SphereRule R, double* __restrict__ vals) {
-  const int n = blockIdx.x * 256 + threadIdx.x;
-  if (n >= R.n_theta * R.n_phi) return;
-  const int i = n / R.n_phi, j = n - i * R.n_phi;
-  const double ct = R.costheta[i], st = sqrt(1.0 - ct * ct), ph = (j + 0.5) * R.dphi;
-  const double q[3] = {R.rex * (st * cos(ph)), R.rex * (st * sin(ph)), R.rex * ct};
-  double v[2];
-  interp2(G, q, v);
-  vals[2 * n] = v[0];
-  vals[2 * n + 1] = v[1];
+  ym[tid] = neville6(yz, cx[1]);
+  __syncthreads();
+  if (a == 0 && want < np) {
+    double y[6];
+#pragma unroll
+    for (int m = 0; m < 6; ++m) y[m] = ym[tid + m];
+    vals[2 * n + f] = neville6(y, cx[0]);
+  }
 }
 
 // One workgroup per mode k = (l, m): every thread sums its points (strided),
@@ -142,7 +145,8 @@ __global__ void __launch_bounds__(256) sphere_modes_kernel(SphereRule R, const d
 
 void launch_sphere_interp(const SphereGrid& G, const SphereRule& R, double* vals, hipStream_t s) {
   const int n = R.n_theta * R.n_phi;
-  if (n > 0) sphere_interp_kernel<<<(n + 255) / 256, 256, 0, s>>>(G, R, vals);
+  if (n > 0)
+    sphere_interp_kernel<<<(n + kSpherePoints - 1) / kSpherePoints, kSpherePer * kSpherePoints, 0, s>>>(G, R, vals);
 }
 
 void launch_sphere_modes(const SphereRule& R, const double* vals, const double* thetap, const int* mode_m,
