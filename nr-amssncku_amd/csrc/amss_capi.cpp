@@ -781,21 +781,31 @@ static void gauss_legendre(int n, double* x, double* w) {
 }
 
 // d^l_{m,s}(theta) of cos(theta): the alternating factorial sum over t
-// (the Wigner formula, e.g. misc.C:271-296).
-static double wigner_d_host(int l, int m, int s, double ct) {
-  auto fact = [](int k) {
-    double f = 1.0;
-    for (int q = 2; q <= k; ++q) f *= q;
-    return f;
-  };
-  const int t0 = std::max(0, m - s), t1 = std::min(l + m, l - s);
-  const double sh = std::sqrt((1.0 - ct) / 2.0), ch = std::sqrt((1.0 + ct) / 2.0);
-  double v = 0.0;
-  for (int t = t0; t <= t1; ++t)
-    v += ((t % 2) ? -1.0 : 1.0) * std::pow(ch, 2 * l + m - s - 2 * t) * std::pow(sh, 2 * t + s - m) /
-         (fact(l + m - t) * fact(l - s - t) * fact(t) * fact(t + s - m));
-  return v * std::sqrt(fact(l + m) * fact(l - m) * fact(l + s) * fact(l - s));
-}
+// (the Wigner formula, e.g. misc.C:271-296), for l up to lmax.  The powers of
+// cos(theta/2) and sin(theta/2) of a node are tabulated once for all its modes
+// (a pow per term, a sine and a cosine per sphere point and seven small copies
+// were 320 of the 740 us of an extraction at 12,800 points and 21 modes).
+struct WignerD {
+  std::vector<double> fact, ch, sh;  // k!, cos(theta/2)^k, sin(theta/2)^k, k <= 2 lmax
+  explicit WignerD(int lmax) : fact(2 * lmax + 1, 1.0), ch(2 * lmax + 1), sh(2 * lmax + 1) {
+    for (int k = 2; k <= 2 * lmax; ++k) fact[k] = fact[k - 1] * k;
+  }
+  void node(double ct) {
+    const double s = std::sqrt((1.0 - ct) / 2.0), c = std::sqrt((1.0 + ct) / 2.0);
+    for (size_t k = 0; k < ch.size(); ++k) {
+      ch[k] = std::pow(c, (int)k);
+      sh[k] = std::pow(s, (int)k);
+    }
+  }
+  double operator()(int l, int m, int s) const {
+    const int t0 = std::max(0, m - s), t1 = std::min(l + m, l - s);
+    double v = 0.0;
+    for (int t = t0; t <= t1; ++t)
+      v += ((t % 2) ? -1.0 : 1.0) * ch[2 * l + m - s - 2 * t] * sh[2 * t + s - m] /
+           (fact[l + m - t] * fact[l - s - t] * fact[t] * fact[t + s - m]);
+    return v * std::sqrt(fact[l + m] * fact[l - m] * fact[l + s] * fact[l - s]);
+  }
+};
 
 struct SurfShim {
   std::mutex mu;
@@ -856,45 +866,53 @@ int amss_surf_wave_dev(const int* ex, const double* X, const double* Y, const do
     hi[a] = C[a][ex[a] - 4] + h / 2;
     cmin[a] = plane ? -2 : 1;
   }
+  std::vector<double> cph(n_phi), sph(n_phi);
+  for (int j = 0; j < n_phi; ++j) {
+    cph[j] = std::cos((j + 0.5) * dphi);
+    sph[j] = std::sin((j + 0.5) * dphi);
+  }
   for (int i = 0; i < n_theta; ++i) {
     const double st = std::sqrt(1.0 - ct[i] * ct[i]);
     for (int j = 0; j < n_phi; ++j) {
-      const double ph = (j + 0.5) * dphi;
-      const double q[3] = {rex * (st * std::cos(ph)), rex * (st * std::sin(ph)), rex * ct[i]};
+      const double q[3] = {rex * (st * cph[j]), rex * (st * sph[j]), rex * ct[i]};
       for (int a = 0; a < 3; ++a)
         if (q[a] < lo[a] || q[a] > hi[a])
           return fail(AMSS_ERR_ARG, std::string(who) + ": the sphere leaves the block's owned cells");
     }
   }
-  // sqrt((2l+1)/4pi) d^l_{m,s} at +cos(theta) and -cos(theta) per mode
-  std::vector<int> mm;
-  std::vector<double> tp;
-  for (int l = spinw; l <= maxl; ++l)
-    for (int m = -l; m <= l; ++m) {
-      mm.push_back(m);
-      for (int sgn = 0; sgn < 2; ++sgn)
-        for (int i = 0; i < n_theta; ++i)
-          tp.push_back(std::sqrt((2 * l + 1.0) / 4.0 / pi) * wigner_d_host(l, m, spinw, sgn ? -ct[i] : ct[i]));
+  // The device's tables, staged in one piece for one copy: coordinates, nodes, weights,
+  // sqrt((2l+1)/4pi) d^l_{m,s} at +cos(theta) and -cos(theta) per mode, then m per mode.
+  const int nm = (maxl + 1) * (maxl + 1) - spinw * spinw, npts = n_theta * n_phi;
+  const size_t ncoord = (size_t)ex[0] + ex[1] + ex[2], ntp = (size_t)nm * 2 * n_theta;
+  const size_t nin = ncoord + 2 * (size_t)n_theta + ntp, nmi = ((size_t)nm + 1) / 2;  // (nmi: nm ints, in doubles)
+  std::vector<double> in(nin + nmi);
+  double* tp = std::copy(wt.begin(), wt.begin() + n_theta,
+                         std::copy(ct.begin(), ct.begin() + n_theta,
+                                   std::copy(Z, Z + ex[2], std::copy(Y, Y + ex[1], std::copy(X, X + ex[0], in.data())))));
+  WignerD wd(maxl);
+  for (int i = 0; i < n_theta; ++i)
+    for (int sgn = 0; sgn < 2; ++sgn) {
+      wd.node(sgn ? -ct[i] : ct[i]);
+      int k = 0;
+      for (int l = spinw; l <= maxl; ++l) {
+        const double norm = std::sqrt((2 * l + 1.0) / 4.0 / pi);
+        for (int m = -l; m <= l; ++m, ++k) tp[((size_t)k * 2 + sgn) * n_theta + i] = norm * wd(l, m, spinw);
+      }
     }
-  const int nm = (int)mm.size(), npts = n_theta * n_phi;
-  const size_t ncoord = (size_t)ex[0] + ex[1] + ex[2];
-  const size_t nd = ncoord + 2 * (size_t)n_theta + tp.size() + 2 * (size_t)npts + 2 * (size_t)nm;
+  int* mm = (int*)(in.data() + nin);
+  for (int l = spinw, k = 0; l <= maxl; ++l)
+    for (int m = -l; m <= l; ++m) mm[k++] = m;
+  const size_t nd = in.size() + 2 * (size_t)npts + 2 * (size_t)nm;
   hipStream_t s = (hipStream_t)stream;
   std::vector<double> out(2 * (size_t)nm);
   {
     std::lock_guard<std::mutex> lk(g_surf.mu);
-    if (int r = g_surf.ensure(nd * sizeof(double) + nm * sizeof(int))) return r;
+    if (int r = g_surf.ensure(nd * sizeof(double))) return r;
     double* d = (double*)g_surf.buf;
     double *dX = d, *dY = dX + ex[0], *dZ = dY + ex[1], *dct = dZ + ex[2], *dwt = dct + n_theta;
-    double *dtp = dwt + n_theta, *dvals = dtp + tp.size(), *dout = dvals + 2 * (size_t)npts;
-    int* dmm = (int*)(dout + 2 * (size_t)nm);
-    HIPCHK(hipMemcpyAsync(dX, X, ex[0] * sizeof(double), hipMemcpyHostToDevice, s));
-    HIPCHK(hipMemcpyAsync(dY, Y, ex[1] * sizeof(double), hipMemcpyHostToDevice, s));
-    HIPCHK(hipMemcpyAsync(dZ, Z, ex[2] * sizeof(double), hipMemcpyHostToDevice, s));
-    HIPCHK(hipMemcpyAsync(dct, ct.data(), n_theta * sizeof(double), hipMemcpyHostToDevice, s));
-    HIPCHK(hipMemcpyAsync(dwt, wt.data(), n_theta * sizeof(double), hipMemcpyHostToDevice, s));
-    HIPCHK(hipMemcpyAsync(dtp, tp.data(), tp.size() * sizeof(double), hipMemcpyHostToDevice, s));
-    HIPCHK(hipMemcpyAsync(dmm, mm.data(), nm * sizeof(int), hipMemcpyHostToDevice, s));
+    double *dtp = dwt + n_theta, *dvals = d + in.size(), *dout = dvals + 2 * (size_t)npts;
+    const int* dmm = (const int*)(d + nin);
+    HIPCHK(hipMemcpyAsync(d, in.data(), in.size() * sizeof(double), hipMemcpyHostToDevice, s));
     SphereGrid G;
     G.rpsi = rpsi;
     G.ipsi = ipsi;
