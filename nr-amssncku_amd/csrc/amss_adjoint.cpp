@@ -139,14 +139,14 @@ void AdjointBlock::fwd_open(const double* const* U, hipStream_t s) {
 
 void AdjointBlock::fwd_stage(int st, double c, double* const* Unext, hipStream_t s) {
   const FieldsIn in = st == 0 ? fin(kY0) : fin(kY + (st - 1) * NFIELD);
-  adj_launch_rhs_k(in, fout(kK), box_, C_, s);
+  const int k = st == 0 ? kAcc : kK;  // sub-step 0's k is where the accumulator starts
+  adj_launch_rhs_k(in, fout(k), box_, C_, s);
   const FieldsOut yn = st < 3 ? fout(kY + st * NFIELD) : (Unext ? as_out(Unext) : fout(kLY));
-  adj_launch_fwd_stage(fin(kY0), fin(kK), fout(kAcc), fout(kZ + st * NFIELD), yn, box_, st, c, tinny_, s);
+  adj_launch_fwd_stage(fin(kY0), fin(k), fout(kAcc), fout(kZ + st * NFIELD), yn, box_, st, c, tinny_, s);
 }
 
 void AdjointBlock::rev_final(const double* const* lam, double c, hipStream_t s) {
-  const FieldsOut lk[4] = {pout(kLK), pout(kLK + NFIELD), pout(kLK + 2 * NFIELD), pout(kLK + 3 * NFIELD)};
-  adj_launch_final(as_in(lam), fin(kZ + 3 * NFIELD), fin(kY0), fout(kLY0), lk, box_, c, tinny_, s);
+  adj_launch_final(as_in(lam), fin(kZ + 3 * NFIELD), fin(kY0), fout(kLY0), pout(kLK + 3 * NFIELD), box_, c, tinny_, s);
 }
 
 void AdjointBlock::rev_rhs(int st, hipStream_t s) {
@@ -160,8 +160,8 @@ void AdjointBlock::rev_rhs(int st, hipStream_t s) {
 }
 
 void AdjointBlock::rev_stage(int st, double c, hipStream_t s) {
-  adj_launch_stage(fin(kLY), fin(kZ + (st - 1) * NFIELD), fin(kY0), fout(kLY0), pout(kLK + (st - 1) * NFIELD),
-                   box_, c, tinny_, s);
+  adj_launch_stage(fin(kLY), fin(kZ + (st - 1) * NFIELD), fin(kY0), fout(kLY0), pin(kLK + 3 * NFIELD),
+                   st == 1 ? 1.0 : 2.0, pout(kLK + (st - 1) * NFIELD), box_, c, tinny_, s);
 }
 
 void AdjointBlock::rev_open(const double* const* U, double* const* lam, hipStream_t s) {

@@ -217,6 +217,10 @@ struct Taps {
   }
 };
 
+// (Bound by the vector L1's load instructions, 335 us at 64^3 points.  Points
+// in 3D tiles for fewer L2 reads: 410-600 us, as rows coalesce worse; every
+// array's tile staged in LDS with its own halo, 23 loads a point instead of 97
+// in two phases of 53 KB: 340-670 us.)
 // dJ/dU(q) = value bar + sum over the output points p whose stencils read q
 // of (stencil weight) x (feature bar at p).  The bars are zero outside the
 // interior and readable 3 planes beyond the array, so they are read at every
@@ -360,47 +364,54 @@ __device__ void enforce_vjp(const double din[6], const double ain[6], double gb[
 }
 
 // Forward stage s of the step at every point:
-//   interior: acc (s = 0: k; 1, 2: += 2k), z = Y0 + c k (s = 3: Y0 + c (k + acc)),
-//             Ynext = LB(z), enforce_ga for s < 3;
+//   interior: acc (s = 0: k, which the RHS kernel has written there; 1, 2: += 2k),
+//             z = Y0 + c k (s = 3: Y0 + c (k + acc)), Ynext = LB(z), enforce_ga for s < 3;
 //   boundary: Ynext = the frozen-ghost fill of Y0 (LB on chi, enforce_ga for s < 3).
+// Of z only what the reverse reads is stored (its masks and enforce_ga's
+// VJP): chi, and for s < 3 the metric and A.  The kernel moves whole arrays:
+// 64^3 points, sub-steps 0-3, 83 us each -> 40 / 68 / 68 / 45 without the
+// other z and sub-step 0's copy of k.
+__host__ __device__ constexpr bool fwd_keeps_z(int stage, int v) {
+  return v == CHI || (stage < 3 && v >= DXX && v <= AZZ);
+}
+template <int STAGE>
 __global__ void __launch_bounds__(256) fwd_stage_kernel(FieldsIn Y0, FieldsIn kk, FieldsOut acc, FieldsOut z,
-                                                        FieldsOut Yn, Box box, int stage, double c, double tinny) {
+                                                        FieldsOut Yn, Box box, double c, double tinny) {
   const long N = (long)box.n[0] * box.n[1] * box.n[2];
   const long q = blockIdx.x * 256L + threadIdx.x;
   if (q >= N) return;
   const int i = (int)(q % box.n[0]), j = (int)((q / box.n[0]) % box.n[1]), k = (int)(q / ((long)box.n[0] * box.n[1]));
   double u[NFIELD];
   if (inside(box, i, j, k)) {
+#pragma unroll
     for (int v = 0; v < NFIELD; ++v) {
       const double kv = kk.p[v][q];
       double w;
-      if (stage == 0) {
-        acc.p[v][q] = kv;
+      if (STAGE == 0) {
         w = Y0.p[v][q] + c * kv;
-      } else if (stage < 3) {
+      } else if (STAGE < 3) {
         acc.p[v][q] = acc.p[v][q] + 2.0 * kv;
         w = Y0.p[v][q] + c * kv;
       } else {
         w = Y0.p[v][q] + c * (kv + acc.p[v][q]);
       }
-      z.p[v][q] = w;
+      if (fwd_keeps_z(STAGE, v)) z.p[v][q] = w;
       u[v] = w;
     }
   } else {
     for (int v = 0; v < NFIELD; ++v) u[v] = Y0.p[v][q];
   }
   u[CHI] = u[CHI] < tinny ? tinny : u[CHI];
-  if (stage < 3) enforce_point(u + DXX, u + AXX);
+  if (STAGE < 3) enforce_point(u + DXX, u + AXX);
   for (int v = 0; v < NFIELD; ++v) Yn.p[v][q] = u[v];
 }
 
 // Reverse of the last combination: lam = dJ/dU^{n+1} ->
-//   interior: lz = lam (chi masked by the lower bound), lY0 = lz,
-//             lk3 = c lz, lk0 = c lz, lk1 = lk2 = 2 c lz;
-//   boundary: lY0 = lam through the stage-3 fill (chi masked), lk = 0.
+//   interior: lz = lam (chi masked by the lower bound), lY0 = lz, lk3 = c lz
+//             (lk0 = lk3 and lk1 = lk2 = 2 lk3 join in adj_stage_kernel);
+//   boundary: lY0 = lam through the stage-3 fill (chi masked); lk stays 0.
 __global__ void __launch_bounds__(256) adj_final_kernel(FieldsIn lam, FieldsIn z3, FieldsIn Y0, FieldsOut lY0,
-                                                        FieldsOut lk0, FieldsOut lk1, FieldsOut lk2, FieldsOut lk3,
-                                                        Box box, double c, double tinny) {
+                                                        FieldsOut lk3, Box box, double c, double tinny) {
   const long N = (long)box.n[0] * box.n[1] * box.n[2];
   const long q = blockIdx.x * 256L + threadIdx.x;
   if (q >= N) return;
@@ -410,18 +421,19 @@ __global__ void __launch_bounds__(256) adj_final_kernel(FieldsIn lam, FieldsIn z
     double l = lam.p[v][q];
     if (v == CHI && (in ? z3.p[CHI][q] : Y0.p[CHI][q]) < tinny) l = 0.0;
     lY0.p[v][q] = l;
-    lk0.p[v][q] = in ? c * l : 0.0;
-    lk1.p[v][q] = in ? 2.0 * c * l : 0.0;
-    lk2.p[v][q] = in ? 2.0 * c * l : 0.0;
-    lk3.p[v][q] = in ? c * l : 0.0;
+    if (in) lk3.p[v][q] = c * l;
   }
 }
 
 // Reverse of stage s < 3 given lY = dJ/dY_{s+1} (RHS adjoint of stage s+1):
-//   interior: Y = E(LB(z)): lz = LB' E'^T lY; lY0 += lz; lk_s += c lz;
+//   interior: Y = E(LB(z)): lz = LB' E'^T lY; lY0 += lz; lk_s = f lk3 + c lz
+//             (f = 1 for s = 0, else 2: the last combination's share, formed
+//             here rather than stored by adj_final_kernel and read back:
+//             95 -> 33 us there at 64^3 points);
 //   boundary: Y = fill(Y0): lY0 += LB' E'(Y0)^T lY.
 __global__ void __launch_bounds__(256) adj_stage_kernel(FieldsIn lY, FieldsIn z, FieldsIn Y0, FieldsOut lY0,
-                                                        FieldsOut lk, Box box, double c, double tinny) {
+                                                        FieldsIn lk3, double f, FieldsOut lk, Box box, double c,
+                                                        double tinny) {
   const long N = (long)box.n[0] * box.n[1] * box.n[2];
   const long q = blockIdx.x * 256L + threadIdx.x;
   if (q >= N) return;
@@ -437,7 +449,7 @@ __global__ void __launch_bounds__(256) adj_stage_kernel(FieldsIn lY, FieldsIn z,
   if (w[CHI] < tinny) l[CHI] = 0.0;
   for (int v = 0; v < NFIELD; ++v) {
     lY0.p[v][q] += l[v];
-    if (in) lk.p[v][q] += c * l[v];
+    if (in) lk.p[v][q] = f * lk3.p[v][q] + c * l[v];
   }
 }
 
@@ -493,18 +505,24 @@ void adj_launch_gather(const FieldsIn& in, const FieldsIn& lam, bool lam_padded,
 }
 void adj_launch_fwd_stage(const FieldsIn& Y0, const FieldsIn& k, const FieldsOut& acc, const FieldsOut& z,
                           const FieldsOut& Yn, const Box& box, int stage, double c, double tinny, hipStream_t s) {
-  const long N = (long)box.n[0] * box.n[1] * box.n[2];
-  fwd_stage_kernel<<<nblk(N), 256, 0, s>>>(Y0, k, acc, z, Yn, box, stage, c, tinny);
+  const unsigned g = nblk((long)box.n[0] * box.n[1] * box.n[2]);
+  switch (stage) {
+    case 0: fwd_stage_kernel<0><<<g, 256, 0, s>>>(Y0, k, acc, z, Yn, box, c, tinny); break;
+    case 1: fwd_stage_kernel<1><<<g, 256, 0, s>>>(Y0, k, acc, z, Yn, box, c, tinny); break;
+    case 2: fwd_stage_kernel<2><<<g, 256, 0, s>>>(Y0, k, acc, z, Yn, box, c, tinny); break;
+    default: fwd_stage_kernel<3><<<g, 256, 0, s>>>(Y0, k, acc, z, Yn, box, c, tinny); break;
+  }
 }
 void adj_launch_final(const FieldsIn& lam, const FieldsIn& z3, const FieldsIn& Y0, const FieldsOut& lY0,
-                      const FieldsOut* lk, const Box& box, double c, double tinny, hipStream_t s) {
+                      const FieldsOut& lk3, const Box& box, double c, double tinny, hipStream_t s) {
   const long N = (long)box.n[0] * box.n[1] * box.n[2];
-  adj_final_kernel<<<nblk(N), 256, 0, s>>>(lam, z3, Y0, lY0, lk[0], lk[1], lk[2], lk[3], box, c, tinny);
+  adj_final_kernel<<<nblk(N), 256, 0, s>>>(lam, z3, Y0, lY0, lk3, box, c, tinny);
 }
 void adj_launch_stage(const FieldsIn& lY, const FieldsIn& z, const FieldsIn& Y0, const FieldsOut& lY0,
-                      const FieldsOut& lk, const Box& box, double c, double tinny, hipStream_t s) {
+                      const FieldsIn& lk3, double f, const FieldsOut& lk, const Box& box, double c, double tinny,
+                      hipStream_t s) {
   const long N = (long)box.n[0] * box.n[1] * box.n[2];
-  adj_stage_kernel<<<nblk(N), 256, 0, s>>>(lY, z, Y0, lY0, lk, box, c, tinny);
+  adj_stage_kernel<<<nblk(N), 256, 0, s>>>(lY, z, Y0, lY0, lk3, f, lk, box, c, tinny);
 }
 void adj_launch_open(const FieldsIn& U, const FieldsIn& lY0, const FieldsOut& lam, long N, hipStream_t s) {
   adj_open_kernel<<<nblk(N), 256, 0, s>>>(U, lY0, lam, N);

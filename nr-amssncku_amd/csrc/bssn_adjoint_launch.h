@@ -20,9 +20,10 @@ void adj_launch_gather(const FieldsIn& in, const FieldsIn& lam, bool lam_padded,
 void adj_launch_fwd_stage(const FieldsIn& Y0, const FieldsIn& k, const FieldsOut& acc, const FieldsOut& z,
                           const FieldsOut& Yn, const Box& box, int stage, double c, double tinny, hipStream_t s);
 void adj_launch_final(const FieldsIn& lam, const FieldsIn& z3, const FieldsIn& Y0, const FieldsOut& lY0,
-                      const FieldsOut* lk, const Box& box, double c, double tinny, hipStream_t s);
+                      const FieldsOut& lk3, const Box& box, double c, double tinny, hipStream_t s);
 void adj_launch_stage(const FieldsIn& lY, const FieldsIn& z, const FieldsIn& Y0, const FieldsOut& lY0,
-                      const FieldsOut& lk, const Box& box, double c, double tinny, hipStream_t s);
+                      const FieldsIn& lk3, double f, const FieldsOut& lk, const Box& box, double c, double tinny,
+                      hipStream_t s);
 void adj_launch_open(const FieldsIn& U, const FieldsIn& lY0, const FieldsOut& lam, long N, hipStream_t s);
 void adj_launch_copy_enforce(const FieldsIn& U, const FieldsOut& Y, long N, hipStream_t s);
 
