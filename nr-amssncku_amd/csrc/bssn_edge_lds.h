@@ -64,6 +64,7 @@ struct EdgeLdsEnv : EdgeStencils<ORD, EdgeLdsEnv<ORD, NRM, ODD, MIRROR>, MIRROR>
       wlo[a] = t.wlo[a];
       if (box.mlo[a] < 0 && wlo[a] < 0) mir |= 1 << a;
     }
+    mir = __builtin_amdgcn_readfirstlane(mir);
     gbase = wlo[0] + wlo[1] * sy + wlo[2] * sz;
     pz = q[2] - wlo[2];
     lt = W::index(q[0] - wlo[0], q[1] - wlo[1], pz, sz, 0);
@@ -97,9 +98,21 @@ struct EdgeLdsEnv : EdgeStencils<ORD, EdgeLdsEnv<ORD, NRM, ODD, MIRROR>, MIRROR>
   // is index m times the parity of v under reflection of a.  The image
   // cells read only cells at or above 0 on the mirrored axes, which this
   // pass does not write.
+  // Its branch and its trip count are the same for every lane (mir is in a
+  // scalar register, the last round is masked).  With mir in a vector register
+  // and a loop that each lane left by itself, the compiler restored the lanes
+  // once, after the branch, and put reloads of spilled registers between the
+  // loop and there, where no lane was active: they loaded nothing.  (Seen in the
+  // assembly of a right-hand-side kernel with this pass, whose A_xz was wrong;
+  // tests/test_lane_masks.py looks for it in every kernel.)  A step of 85 x 61 x 45
+  // interior points above a plane, copy boundary: 1,448 us with that loop, 1,399
+  // with this one.
   __device__ __forceinline__ void mirror(int v, lds_double* b) const {
     const int ob = odd_base(v);
-    for (int c = tid; c < W::W0 * W::W1 * W::W2; c += kEdgeThreads) {
+    constexpr int kCells = W::W0 * W::W1 * W::W2;
+#pragma unroll 1
+    for (int c0 = 0; c0 < kCells; c0 += kEdgeThreads) {
+      const int c = c0 + tid;
       const int x[3] = {c % W::W0, (c / W::W0) % W::W1, c / (W::W0 * W::W1)};
       int m[3];
       double s = 1.0;
@@ -113,7 +126,8 @@ struct EdgeLdsEnv : EdgeStencils<ORD, EdgeLdsEnv<ORD, NRM, ODD, MIRROR>, MIRROR>
           img = true;
         }
       }
-      if (img) b[W::index(x[0], x[1], x[2], sz, ob)] = s * b[W::index(m[0] - wlo[0], m[1] - wlo[1], m[2] - wlo[2], sz, ob)];
+      if (img && c < kCells)
+        b[W::index(x[0], x[1], x[2], sz, ob)] = s * b[W::index(m[0] - wlo[0], m[1] - wlo[1], m[2] - wlo[2], sz, ob)];
     }
   }
   __device__ __forceinline__ lds_double* slot(int grp) const { return buf + (grp & 1) * W::PAD; }
@@ -222,7 +236,7 @@ __device__ __forceinline__ void edge_rhs_tile(const FieldsIn& in, const AuxOut& 
 // and barrier after another; separate launches would queue these chains).
 // Bound by those chains and by VALU issue.  MIRROR is a variant of its own
 // because the mirror pass and the dissipation's branch cut the point
-// computation into blocks, and its registers spill: 1,020 bytes of scratch per
+// computation into blocks, and its registers spill: 1,068 bytes of scratch per
 // lane with them, 360 without; all tiles of a 134^3 patch 503 -> 442 us beside
 // the interior, of 70^3 and 76^3 patches 208 -> 183.  An odd-pitched patch took
 // the direct kernel before: a step of 85 x 61 x 45 interior points with the

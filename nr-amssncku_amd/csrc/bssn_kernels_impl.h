@@ -307,8 +307,8 @@ template <int G, bool CO, bool ODD>
 void launch_rhs_lds(const FieldsIn& in, const FieldsIn& mat, const FieldsOut& out, const AuxOut& aux, const Box& box,
                     const Coef& C, int* flag, hipStream_t s);
 
-// Whether it may run: no symmetry plane (the variant with the mirror pass,
-// whose point computations spilled most, gave wrong values and was not kept),
+// Whether it may run: no symmetry plane (a variant with the mirror pass gave
+// wrong values, for the reason told at EdgeLdsEnv::mirror, and was not kept),
 // every axis of 5 points or more (the boundary tiles' windows are laid out
 // for those), 32-bit byte offsets, and with an even row
 // pitch every state array on 16 bytes (the direct loads' alignment; with an
