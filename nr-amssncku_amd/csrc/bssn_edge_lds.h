@@ -82,7 +82,7 @@ struct EdgeLdsEnv : EdgeStencils<ORD, EdgeLdsEnv<ORD, NRM, ODD, MIRROR>, MIRROR>
     for (int r = 0; r < W::ROUNDS; ++r) {
       int x, y, z;
       W::element(2 * (r * kEdgeThreads + tid), sz, ob, x, y, z);
-      const int gi = W::clamp(gbase + x + y * sy + z * sz, gmax);
+      const int gi = W::clamp(gbase + x + y * sy + z * sz, gmax, MIRROR);
       __builtin_amdgcn_global_load_lds((__attribute__((address_space(1))) void*)(base + gi),
                                        (__attribute__((address_space(3))) void*)(b + 2 * (r * kEdgeThreads + wave * 64)),
                                        16, 0, 0);
@@ -113,20 +113,13 @@ struct EdgeLdsEnv : EdgeStencils<ORD, EdgeLdsEnv<ORD, NRM, ODD, MIRROR>, MIRROR>
 #pragma unroll 1
     for (int c0 = 0; c0 < kCells; c0 += kEdgeThreads) {
       const int c = c0 + tid;
-      const int x[3] = {c % W::W0, (c / W::W0) % W::W1, c / (W::W0 * W::W1)};
-      int m[3];
+      int x[3], m[3];
+      const int im = W::image(c, wlo, mir, x, m);
       double s = 1.0;
-      bool img = false;
 #pragma unroll
-      for (int a = 0; a < 3; ++a) {
-        m[a] = wlo[a] + x[a];
-        if (((mir >> a) & 1) && m[a] < 0) {
-          m[a] = -m[a] - 1;
-          s *= parity(v, a);
-          img = true;
-        }
-      }
-      if (img && c < kCells)
+      for (int a = 0; a < 3; ++a)
+        if ((im >> a) & 1) s *= parity(v, a);
+      if (im != 0 && c < kCells)
         b[W::index(x[0], x[1], x[2], sz, ob)] = s * b[W::index(m[0] - wlo[0], m[1] - wlo[1], m[2] - wlo[2], sz, ob)];
     }
   }

@@ -148,14 +148,35 @@ struct EdgeWindow {
       z = e / P01;
     }
   }
-  // Array index gi of a chunk's first element, clamped to the chunks that hold
-  // one of the array's N elements.  ODD: gi has the parity its 16-byte
-  // alignment needs; the first (last) chunk may reach one element before
-  // (past) the array, inside the same 16 bytes as its first (last) element.
-  AMSS_HD static int clamp(int gi, int N) {
-    const int lo = ODD ? -(gi & 1) : 0, hi = ODD ? N - 1 - ((gi ^ (N - 1)) & 1) : N - 2;
+  // Array index gi of a chunk's first element, clamped to the chunks inside
+  // the array of N elements.  ODD: gi keeps the parity its 16-byte alignment
+  // needs, so element N - 1, and element 0 of an array that starts off 16 bytes,
+  // may have no chunk left.  No stencil reads them: a point of these shells is
+  // inside the outermost layer on every axis and a stencil moves along two axes
+  // at most.  Only next to a symmetry plane is element 0 read (planes); its
+  // chunk then starts on the element before the array, which is the last of
+  // the preceding field in the Block's slab (the slab itself starts on 16 bytes).
+  AMSS_HD static int clamp(int gi, int N, bool planes = true) {
+    const int lo = ODD ? (planes ? -(gi & 1) : gi & 1) : 0, hi = ODD ? N - 2 - ((gi ^ N) & 1) : N - 2;
     gi = gi < lo ? lo : gi;
     return gi > hi ? hi : gi;
+  }
+  // Window element x of cell c in the window at wlo, and the array index m it
+  // holds: itself, or its mirror -m - 1 on each axis where it lies below a
+  // symmetry plane (the axes of mir; the result's bits say which).
+  AMSS_HD static int image(int c, const int wlo[3], int mir, int x[3], int m[3]) {
+    x[0] = c % W0;
+    x[1] = (c / W0) % W1;
+    x[2] = c / (W0 * W1);
+    int im = 0;
+    for (int a = 0; a < 3; ++a) {
+      m[a] = wlo[a] + x[a];
+      if (((mir >> a) & 1) && m[a] < 0) {
+        m[a] = -m[a] - 1;
+        im |= 1 << a;
+      }
+    }
+    return im;
   }
 };
 
