@@ -101,6 +101,15 @@ AMSS_HD EdgeShells edge_shells_of(const int n[3], const int lo[3], const int hi[
   return EdgeShells{{Shell(z, n, L1, H1), Shell(L1, H1, L2, H2), Shell(L2, H2, blo, bhi)}};
 }
 
+// The boundary stencils' reads in global memory (EdgeEnv, bssn_env.h), one
+// axis at a time.  A read below index 0 is served by the mirror image of the
+// first points for every Symmetry (the reference's symmetry_bd).  The upwind
+// stencil takes all seven samples at offsets m within +-3 whatever room the
+// array has; those past the upper end, which go unused, read the last point.
+// Every axis has 5 points, or 3 with a symmetry plane, so both stay inside.
+AMSS_HD int edge_fold(int q) { return q < 0 ? -q - 1 : q; }
+AMSS_HD int edge_clamp(int pos, int m, int n) { return m < n - 1 - pos ? m : n - 1 - pos; }
+
 constexpr int kEdgeTile = 16;                        // points per in-plane tile axis
 constexpr int kEdgeThreads = kEdgeTile * kEdgeTile;  // one point per thread
 

@@ -1,6 +1,7 @@
 // bssn_env.h -- stencil environments and result sinks for bssn_rhs_point.
 #pragma once
 #include "bssn_algebra.h"
+#include "bssn_edge_tiles.h"
 
 namespace amss {
 
@@ -252,16 +253,15 @@ struct EdgeEnv : EdgeStencils<ORD, EdgeEnv<ORD>> {
   __device__ double rel(int v, int di, int dj, int dk, double off) const {
     int a = this->i + di, b = this->j + dj, c = this->k + dk;
     double s = 1.0;
-    if (a < 0) { a = -a - 1; s *= parity(v, 0); }
-    if (b < 0) { b = -b - 1; s *= parity(v, 1); }
-    if (c < 0) { c = -c - 1; s *= parity(v, 2); }
+    if (a < 0) { a = edge_fold(a); s *= parity(v, 0); }
+    if (b < 0) { b = edge_fold(b); s *= parity(v, 1); }
+    if (c < 0) { c = edge_fold(c); s *= parity(v, 2); }
     return (F.p[v][a + b * sy + c * sz] + off) * s;
   }
-  // rel with the index clamped to the array's last point: inside the array
-  // for every offset within +-3 (a mirrored index is at most 2)
+  // rel with the index clamped to the array's last point
   __device__ double rel_clamped(int v, int di, int dj, int dk, double off) const {
-    return rel(v, min(di, this->n[0] - 1 - this->i), min(dj, this->n[1] - 1 - this->j), min(dk, this->n[2] - 1 - this->k),
-               off);
+    return rel(v, edge_clamp(this->i, di, this->n[0]), edge_clamp(this->j, dj, this->n[1]),
+               edge_clamp(this->k, dk, this->n[2]), off);
   }
   __device__ double val(int v) const { return F.p[v][this->i + this->j * sy + this->k * sz]; }
   __device__ double mat(int m) const { return M.p[m][this->i + this->j * sy + this->k * sz]; }
