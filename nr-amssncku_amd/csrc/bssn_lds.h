@@ -105,12 +105,8 @@ __device__ __forceinline__ BufIo tile_io(int i, int j, int k, int hx, int hy, in
 #ifndef AMSS_LDS_FENCE
 #define AMSS_LDS_FENCE 1
 #endif
-#ifndef AMSS_LDS_PAIRS
-#define AMSS_LDS_PAIRS 1
-#endif
-// LDS tile buffers per workgroup: two pairs (two field groups per barrier)
-// or two single buffers.
-constexpr int kLdsBuffers = AMSS_LDS_PAIRS ? 4 : 2;
+// LDS tile buffers per workgroup: two pairs (two field groups per barrier).
+constexpr int kLdsBuffers = 4;
 
 // Doubles of the epilogue's stash (LdsRk4) behind a kernel's tile buffers of
 // npad doubles each, for workgroups of `points` threads: 6 per thread, or none
@@ -120,12 +116,9 @@ constexpr int lds_stash(int points, int npad) {
   return (512 / points) * (kLdsBuffers * npad + 6 * points) * 8 <= 160 * 1024 ? 6 * points : 0;
 }
 
-#ifndef AMSS_TOP
-#define AMSS_TOP 1
-#endif
-// When a pair's two halo tiles are issued, one pair ahead: both at the barrier
-// (0), the first there and the second with the second group (1), both with the
-// second group (2).  Self::kDmaAt says; 1 by default.
+// When a pair's two halo tiles are issued, one pair ahead: the first at the
+// barrier and the second with the second group (1), both with the second group
+// (2).  Self::kDmaAt says; 1 by default.
 template <class S, class = void>
 struct DmaAt {
   static constexpr int v = 1;
@@ -201,7 +194,6 @@ struct LdsEnv {
   // Groups are staged two at a time: groups 2q and 2q+1 share pair q & 1,
   // so a tile needs one barrier per two field groups.
   __device__ __forceinline__ lds_double* slot(int grp) const {
-    if (!AMSS_LDS_PAIRS) return (grp & 1) ? buf1 : buf0;
     return (((grp >> 1) & 1) ? buf1 : buf0) + (grp & 1) * T::NPAD;
   }
   __device__ __forceinline__ lds_double* cur() const { return slot(g - 1); }  // g already advanced
@@ -231,33 +223,24 @@ struct LdsEnv {
     return v == CHI || v == TRK || v == LAP || (v >= DXX && v <= AZZ) || (v >= BETAX && v <= BETAX + 2);
   }
   __device__ __forceinline__ void prologue() {
-    if (AMSS_TOP) {
 #pragma unroll
-      for (int v = 0; v < NFIELD; ++v)
-        if (in_top(v)) top[v] = at_p.ld(F.ptr(v));
-    }
-    if (AMSS_LDS_PAIRS) ahead(0);
+    for (int v = 0; v < NFIELD; ++v)
+      if (in_top(v)) top[v] = at_p.ld(F.ptr(v));
+    ahead(0);
     __builtin_amdgcn_sched_barrier(0);
     issue(group_field(0), slot(0));
-    if (AMSS_LDS_PAIRS) issue(group_field(1), slot(1));
+    issue(group_field(1), slot(1));
   }
   __device__ __forceinline__ void begin(int v) {
     constexpr int kAt = DmaAt<Self>::v;
-    if (!AMSS_LDS_PAIRS) {
-      __builtin_amdgcn_s_waitcnt(0);
-      __syncthreads();
-      if (g + 1 < NFIELD) issue(group_field(g + 1), slot(g + 1));
-    } else if ((g & 1) == 0) {
+    if ((g & 1) == 0) {
       __builtin_amdgcn_s_waitcnt(0);  // this wave's DMA of groups g, g+1 (and everything else) landed
       __syncthreads();                // ... for every wave; and the readers of groups g-2, g-1 are done
       rotate();
       if (g + 2 < NFIELD) ahead(g + 2);
       __builtin_amdgcn_sched_barrier(0);
-      if (g + 2 < NFIELD) {
-        if (kAt < 2) issue(group_field(g + 2), slot(g + 2));
-        if (kAt < 1) issue(group_field(g + 3), slot(g + 3));
-      }
-    } else if (kAt > 0 && g + 1 < NFIELD) {
+      if (kAt < 2 && g + 2 < NFIELD) issue(group_field(g + 2), slot(g + 2));
+    } else if (g + 1 < NFIELD) {
       // the next pair's halo loads start with the pair's second group
       __builtin_amdgcn_sched_barrier(0);
       if (kAt > 1) issue(group_field(g + 1), slot(g + 1));
@@ -288,7 +271,7 @@ struct LdsEnv {
   // the centre value of the open group's field is in its halo tile; the
   // pair's extra centre values were loaded at its barrier
   __device__ __forceinline__ double val(int v) const {
-    if (AMSS_TOP && g == 0 && in_top(v)) return top[v];
+    if (g == 0 && in_top(v)) return top[v];
     if (g > 0 && v == group_field(g - 1)) return at(v, 0);
     if (v == xf[0]) return xv[0];
     if (v == xf[1]) return xv[1];
