@@ -69,9 +69,10 @@ int xfer_plan(const double* llbc, const double* uubc, const int* extc, const dou
 // from registers; y and x follow through LDS the same way.  Bound by the
 // latency of one such round trip per tile (an 8-16 deep chain of loads, two
 // barriers) and by the launch, not by bytes: the earlier kernels staged the
-// block in LDS in a loop whose every load waited.  A 134^3 fine array takes
-// 12.9 us (36 before; its 9 bytes a cell 3.8 us at the rate of a copy), 62^3
-// coarse cells 11.4 us (28).
+// block in LDS in a loop whose every load waited.  Over 24 fields in turn a
+// 134^3 fine array takes 12.9 us (36 before; its 9 bytes a cell 3.8 us at the
+// rate of a copy), 61^3 coarse cells 11.4 us (28); the same arrays again and
+// again, 11.0 us and (62^3 cells) 8.5.
 // blockIdx.y is the field, blockIdx.x a tile of one of the regions.
 // Source cells past what the valid target cells read are clamped or skipped;
 // cells past the end of the target range are not stored.

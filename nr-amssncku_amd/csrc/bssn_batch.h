@@ -96,6 +96,12 @@ struct FillWork {
 // row touches whole cache lines where an 8-point one straddles two
 // (lds_tile_shape has the figures).  Both in one launch, a branch per tile, cost
 // 60 bytes of scratch per lane: 37 patches 21.1 ms against 20.5.
+// kWideFill is 32 points at the wide tile's 0.84 of a cube's time per point:
+// fewer points than that cost less in cubes, if cubes padded nothing.  They do:
+// the four sub-steps of x 96 x 96 points take, in cubes / with a last wide tile,
+// 456 / 528 us for x = 24 and 1,178 / 1,023 for 32 + 24 (below the line), 606 /
+// 536 for 26 and 1,332 / 1,022 for 32 + 26 (below it, where the wide tile would
+// be better), 640 / 558 for 28 and 1,373 / 1,048 for 32 + 28 (above it).
 constexpr int kWideX = 32, kWideYZ = 4, kWideFill = 27;
 constexpr int kNumTileShapes = 4;
 __host__ __device__ constexpr int tile_dim(int shape, int a) {

@@ -53,10 +53,10 @@ __host__ __device__ constexpr int tile_row(int r, int TY) { return TY == 8 ? ((r
 //  ODD pitch: rows one double longer (elements x = -1 .. TX + 5; -1 is padding
 //    whose chunk may hold it and x = 0), planes of an even pitch with room for
 //    one more; where the arrays' plane pitch is odd too, odd planes start one
-//    double later.  A sub-step of 85^3 points takes 395 us on 8x8x8 tiles (the
-//    direct kernel, which took odd pitches before, about 650); the same tiles
-//    filled by 4-byte loads spilled scalar registers (730 us with the
-//    residuals).
+//    double later.  A sub-step of 85^3 points takes 376 us on 8x8x8 tiles and
+//    311 on 32x4x4 ones, which lds_tile_shape picks there (the direct kernel,
+//    which took odd pitches before, about 650); 8x8x8 tiles filled by 4-byte
+//    loads spilled scalar registers (730 us with the residuals).
 // LDS banks: a ds_read_b64 serves 16 lanes at a time.  Rows of 16 points or
 // more need no care; an 8-point row pairs with one 16 banks away: row y + 4
 // (EVEN, tile_row), or the same row of plane z + 1 (ODD: planes of 216
@@ -346,8 +346,9 @@ struct LdsEnv {
 // 1,151), and so do the tile lists (18.1 -> 18.3 ms).
 // Non-temporal traffic (WIDE_NT, wide tiles): what a sub-step writes, and what
 // a corrector reads of the old state and the accumulator, is not touched
-// again before the next sub-step, and wide tiles are used on boxes whose 24
-// fields exceed the caches; marked so, it leaves the L2 to the halo tiles.
+// again before the next sub-step, and wide tiles are used on boxes of more than
+// 262,144 points, whose 24 fields (50 MB) exceed the L2s; marked so, it leaves
+// them to the halo tiles.
 // The predictor's old state IS the field its halo tiles are filled from, so
 // its loads stay plain.  128^3 points, sub-steps 0-3 (residuals in 0):
 // 1081 / 932 / 906 / 768 -> 1014 / 916 / 892 / 764 us.  72^3 points on

@@ -8,16 +8,19 @@ namespace amss {
 
 // The tile shape for an interior box.  4-deep 8x8 tiles (256 threads, two
 // workgroups per CU) spread a small box over more CUs and end it sooner: up to
-// two rounds of 512-point tiles on the chip's 256 CUs (per sub-step of n^3
-// points against 8x8x8, 32 against 42 us at 16^3, 37 against 46 at 32^3, 92
-// against 103 at 56^3 with 343 tiles, 132 against 139 at 64^3 with 512; the
-// other way 526 against 496 at 96^3 with 1728).  Above, rows of 32 points where
+// two rounds of 512-point tiles on the chip's 256 CUs (mean sub-step of n^3
+// points against 8x8x8, 31 against 42 us at 16^3, 36 against 45 at 32^3, 90
+// against 99 at 56^3 with 343 tiles, 123 against 122 at 64^3 with 512; the
+// other way 489 against 457 at 96^3 with 1728).  Above, rows of 32 points where
 // the box does not pad them away: their loads and stores touch whole cache
 // lines (an 8-point row of an array whose rows are not 64-byte aligned touches
 // two, half of each), which is worth more than the smaller halo of a cube:
-// sub-steps 0-3 of 128^3 points take 1,070 / 921 / 894 / 762 us against 1,230 /
-// 1,138 / 1,102 / 927, 0.84 of the time per point on average, so a 32x4x4 cover
-// may hold 1/0.84 of the cubic one's points.
+// sub-steps 0-3 of 128^3 points take 1,004 / 875 / 851 / 759 us against 1,207 /
+// 1,077 / 1,036 / 921, 0.82 of the time per computed point (96^3 0.83, 85^3
+// 0.76, 72^3 and 80^3 0.80-0.81, 90 x 64 x 64 0.85); the line lies at 0.84, what it was when
+// the wide tiles were new, so a 32x4x4 cover may hold 1/0.84 of the cubic
+// one's points.  At the line, 80^3 (1.20 times the points) takes 255 us wide
+// and 261 cubic; 72^3 (1.33) 202 and 189.
 inline int lds_tile_shape(const Box& box) {
   long n[3];  // points the cover by each shape computes
   for (int s = 0; s < 3; ++s) {
