@@ -77,12 +77,12 @@ struct EdgeLdsEnv : EdgeStencils<ORD, EdgeLdsEnv<ORD, NRM, ODD, MIRROR>, MIRROR>
   __device__ __forceinline__ void issue(int v, lds_double* b) const {
     const auto base = F.ptr(v);
     const int wave = tid >> 6;
-    const int ob = odd_base(v);
+    const int ob = odd_base(v), par = ODD ? (int)((uintptr_t)base >> 3) & 1 : 0;
 #pragma unroll
     for (int r = 0; r < W::ROUNDS; ++r) {
       int x, y, z;
       W::element(2 * (r * kEdgeThreads + tid), sz, ob, x, y, z);
-      const int gi = W::clamp(gbase + x + y * sy + z * sz, gmax, MIRROR);
+      const int gi = W::clamp(gbase + x + y * sy + z * sz, gmax, MIRROR, par);
       __builtin_amdgcn_global_load_lds((__attribute__((address_space(1))) void*)(base + gi),
                                        (__attribute__((address_space(3))) void*)(b + 2 * (r * kEdgeThreads + wave * 64)),
                                        16, 0, 0);

@@ -165,11 +165,13 @@ struct EdgeWindow {
   // at most.  Only next to a symmetry plane is element 0 read (planes); its
   // chunk then starts on the element before the array, which is the last of
   // the preceding field in the Block's slab (the slab itself starts on 16 bytes).
-  AMSS_HD static int clamp(int gi, int N, bool planes = true) {
-    const int lo = ODD ? (planes ? -(gi & 1) : gi & 1) : 0, hi = ODD ? N - 2 - ((gi ^ N) & 1) : N - 2;
+  // p: gi's parity, the same for every chunk of a field.
+  AMSS_HD static int clamp(int gi, int N, bool planes, int p) {
+    const int lo = ODD ? (planes ? -p : p) : 0, hi = ODD ? N - 2 - ((p ^ N) & 1) : N - 2;
     gi = gi < lo ? lo : gi;
     return gi > hi ? hi : gi;
   }
+  AMSS_HD static int clamp(int gi, int N, bool planes = true) { return clamp(gi, N, planes, gi & 1); }
   // Window element x of cell c in the window at wlo, and the array index m it
   // holds: itself, or its mirror -m - 1 on each axis where it lies below a
   // symmetry plane (the axes of mir; the result's bits say which).
