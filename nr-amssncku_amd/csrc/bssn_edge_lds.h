@@ -229,7 +229,7 @@ __device__ __forceinline__ void edge_rhs_tile(const FieldsIn& in, const AuxOut& 
 // and barrier after another; separate launches would queue these chains).
 // Bound by those chains and by VALU issue.  MIRROR is a variant of its own
 // because the mirror pass and the dissipation's branch cut the point
-// computation into blocks, and its registers spill: 1,068 bytes of scratch per
+// computation into blocks, and its registers spill: 1,048 bytes of scratch per
 // lane with them, 360 without; all tiles of a 134^3 patch 503 -> 442 us beside
 // the interior, of 70^3 and 76^3 patches 208 -> 183.  An odd-pitched patch took
 // the direct kernel before: a step of 85 x 61 x 45 interior points with the
